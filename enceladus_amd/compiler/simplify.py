@@ -1,7 +1,8 @@
 """The simplifier: constant folding, algebraic identities, loop-invariant hoisting, common
 subexpressions and dead code (reference: compiler/passes/simplify.py:336-511).
 
-`simplify(fn)` repeats four rewrites until none applies (at most a few rounds):
+`simplify(fn)` first replaces arguments known to be 1 with the constant
+(`specialize_ones`), then repeats four rewrites until none applies (at most a few rounds):
 
 - **fold**: an elementwise op (`binary`, `unary`, `cast`, `select`) whose operands are all
   constant becomes a constant, evaluated by `compiler.fold` with the interpreter's
@@ -226,8 +227,27 @@ class _Rewriter:
                 self._finish(r)
 
 
+def specialize_ones(fn: ir.Func) -> None:
+    """Replaces integer arguments that this specialization knows to be 1 (`equal_to_1`, part
+    of the launch key) with the constant, so that a stride of 1 folds away: the axis analysis
+    then sees the dimension it multiplies as contiguous."""
+    ones, consts = {}, []
+    for a in fn.args:
+        if a.facts.get("equal_to_1") and isinstance(a.type, ir.TType) and a.type.is_scalar and \
+                not a.type.ptr and a.type.dtype.is_int() and not a.type.dtype.is_bool():
+            c = ir.Op("const", [], [a.type], {"value": 1})
+            consts.append(c)
+            ones[a.id] = c.result
+    if not ones:
+        return
+    for op in ir.walk(fn.body):
+        op.operands = [ones.get(o.id, o) for o in op.operands]
+    fn.body.ops[:0] = consts
+
+
 def simplify(fn: ir.Func, rounds: int = 4) -> None:
     """Rewrites `fn` in place (see the module docstring)."""
+    specialize_ones(fn)
     for _ in range(rounds):
         rw = _Rewriter(fn)
         changed = rw.run()
