@@ -232,21 +232,34 @@ class Emitter:
         for d in range(len(shape)):
             if info.contig[d] > info.contig[best]:
                 best = d
-        vec = min(info.contig[best], max(1, info.div[best] // es), max(1, 16 // es),
-                  shape[best])
+        vec = min(info.contig[best], max(1, 16 // es), shape[best])
+        if ptr.type.numel < self.nt * vec:
+            # a tile too small to give every thread such a vector keeps to its alignment:
+            # wider ones would only leave more threads with copies
+            vec = min(vec, max(1, info.div[best] // es))
         vec = 1 << LY.log2(max(1, vec))
         order = [best] + [d for d in reversed(range(len(shape))) if d != best]
         return LY.blocked(shape, order, vec, self.nw)
 
     def mem_vec(self, ptr: ir.Value, lay: LY.Layout) -> int:
-        """Elements per vector access for `ptr` read in `lay` (contiguity, alignment)."""
+        """Elements per vector access for `ptr` read in `lay`: the run that is contiguous in
+        memory, up to 16 bytes. Alignment does not limit it: gfx950 runs global vector
+        accesses at any element alignment (`vec_suffix` picks the form that says so), and one
+        16-byte access per lane beats several narrow ones however it is aligned."""
         info = self.axis.get(ptr)
         es = ptr.type.dtype.itemsize
         d, nb = lay.vec_dim_bits()
         if not lay.reg or nb == 0:
             return 1
-        v = min(1 << nb, info.contig[d], max(1, info.div[d] // es), max(1, 16 // es))
+        v = min(1 << nb, info.contig[d], max(1, 16 // es))
         return 1 << LY.log2(max(1, v))
+
+    def vec_suffix(self, ptr: ir.Value, lay: LY.Layout, V: int) -> str:
+        """"" when `ptr`'s V-element vectors in `lay` are known to be aligned to their size,
+        "_u" (the element-aligned accessors) otherwise."""
+        d, _ = lay.vec_dim_bits()
+        es = ptr.type.dtype.itemsize
+        return "" if V == 1 or self.axis.get(ptr).div[d] >= V * es else "_u"
 
     def wave_run_bytes(self, ptr: ir.Value, lay: LY.Layout) -> int:
         """Bytes one vector access of `ptr` in `lay` covers contiguously across a wave:
@@ -1254,7 +1267,9 @@ class Emitter:
         self.emit(f"{t} {nm}[{lay.nregs}];")
         hdr = f"for (int rv = 0; rv < {lay.nregs}; rv += {V}) {{"
         pe = lambda i: self.elem(ptr, lay, f"rv + {i}" if i else "rv")  # noqa: E731
-        ld = "vload_nt" if self._streaming_load(op) else "vload"
+        streaming = self._streaming_load(op)
+        sfx = self.vec_suffix(ptr, lay, V)
+        ld = "vload_nt" if streaming and not sfx else "vload" + sfx
 
         def plain():
             self.emit("#pragma unroll")
@@ -1270,7 +1285,7 @@ class Emitter:
         # (e.g. offs < n away from the last program) gets a branch-free unmasked path.
         cond = None if self.opt.get("no_edge_versioning") else self.all_true(mask)
         if cond and self._assume(cond):
-            if ld == "vload_nt" and not self.opt.get("no_serial_streams"):
+            if streaming and not self.opt.get("no_serial_streams"):
                 # One streaming tile load in flight per wave: waiting for the previous one
                 # before issuing the next measured +1.5% on vector add (two 1 GiB inputs).
                 if self.fast_streams:
@@ -1287,21 +1302,147 @@ class Emitter:
             self.emit("} else {")
         me = lambda i: self.elem(mask, lay, f"rv + {i}" if i else "rv")  # noqa: E731
         oe = lambda i: self.elem(other, lay, f"rv + {i}" if i else "rv")  # noqa: E731
-        self.emit("#pragma unroll")
-        self.emit(hdr)
-        if V > 1:
-            allm = " && ".join(f"({me(i)})" for i in range(V))
-            self.emit(f"  if ({allm}) {{ ek::{ld}<{t}, {V}>(&{nm}[rv], {pe(0)}); }}")
-            self.emit("  else {")
+        dv = lay.vec_dim_bits()[0]
+        edge = self._edge_bounds(mask, lay) if V > 1 and self.kind.get(ptr.id) == "cheap" and \
+            self.axis.get(ptr).contig[dv] == lay.shape[dv] else None
+        if edge is not None:
+            self._clamped_load(op, lay, V, nm, edge)
+        elif V > 1:
+            # Whole vectors load first, partly selected ones element by element after them: a
+            # load under an `if` without an `else` goes straight to its registers, so a
+            # thread's vectors are in flight together.
+            allm, anym = self._vec_mask(mask, lay, V)
+            self.emit("#pragma unroll")
+            self.emit(f"for (int rv = 0; rv < {lay.nregs}; ++rv) {nm}[rv] = {oe(0)};")
+            self.emit("#pragma unroll")
+            self.emit(hdr)
+            self.emit(f"  if ({allm}) ek::{ld}<{t}, {V}>(&{nm}[rv], {pe(0)});")
+            self.emit("}")
+            self.emit("#pragma unroll")
+            self.emit(hdr)
+            self.emit(f"  if (({anym}) && !({allm})) {{")
             for i in range(V):
-                self.emit(f"    {nm}[rv + {i}] = ({me(i)}) ? *({pe(i)}) : {oe(i)};")
+                self.emit(f"    if ({me(i)}) {nm}[rv + {i}] = *({pe(i)});")
             self.emit("  }")
+            self.emit("}")
         else:
+            self.emit("#pragma unroll")
+            self.emit(hdr)
             self.emit(f"  {nm}[rv] = ({me(0)}) ? *({pe(0)}) : {oe(0)};")
-        self.emit("}")
+            self.emit("}")
         if cond:
             self.emit("}")
         self.define(res, nm)
+
+    def _mask_terms(self, mask: ir.Value, rank: int):
+        """The conjunction `mask` as [(term, dim, x, bound, inclusive)]: the mask is the AND of
+        its terms, each `x < bound` (`<=` when inclusive) with x counting up by one along the
+        whole of dimension `dim` and equal along the others, and the bound one value for the
+        tile; or None when some term has another form."""
+        op = mask.op
+        if op is None:
+            return None
+        if op.name == "binary" and op.attrs["op"] == "and":
+            a, b = (self._mask_terms(o, rank) for o in op.operands)
+            return None if a is None or b is None else a + b
+        v = mask
+        while v.op is not None and v.op.name == "broadcast" and \
+                len(v.op.operands[0].type.shape) == rank:
+            v = v.op.operands[0]
+        o = v.op
+        if o is None or o.name != "binary" or o.attrs["op"] not in ("lt", "le", "gt", "ge") or \
+                len(v.type.shape) != rank:
+            return None
+        x, bound = o.operands if o.attrs["op"] in ("lt", "le") else o.operands[::-1]
+        if x.type.ptr or x.type.dtype not in (core.int32, core.int64) or any(
+                self.kind.get(q.id) != "cheap" for q in (x, bound)):
+            return None
+        shape, ix, ib = v.type.shape, self.axis.get(x), self.axis.get(bound)
+        if any(ib.const[d] != shape[d] for d in range(rank)):
+            return None
+        dims = [d for d in range(rank) if shape[d] > 1 and ix.const[d] != shape[d]]
+        if len(dims) != 1 or ix.contig[dims[0]] != shape[dims[0]]:
+            return None
+        return [(mask, dims[0], x, bound, o.attrs["op"] in ("le", "ge"))]
+
+    def _vec_mask(self, mask: ir.Value, lay: LY.Layout, V: int) -> tuple[str, str]:
+        """(all, any): conditions over the V mask elements at register `rv` of `lay`. A
+        conjunction of upper bounds selects a prefix of the vector, so its last element
+        decides `all` and its first `any`; other masks are tested element by element."""
+        elem = lambda i: f"({self.elem(mask, lay, f'rv + {i}' if i else 'rv')})"  # noqa: E731
+        if self._mask_terms(mask, len(lay.shape)) is not None:
+            return elem(V - 1), elem(0)
+        return " && ".join(map(elem, range(V))), " || ".join(map(elem, range(V)))
+
+    def _edge_bounds(self, mask: ir.Value, lay: LY.Layout):
+        """Per dimension, the C++ expression (int64) of how many leading coordinates of the
+        tile `mask` selects, None for an unbounded dimension; None overall when the mask is
+        no such box."""
+        rank = len(lay.shape)
+        terms = self._mask_terms(mask, rank)
+        if terms is None:
+            return None
+        out: list = [None] * rank
+        for _, d, x, bound, incl in terms:
+            z = ["0"] * rank
+            e = f"((int64_t){self.cheap(bound, z)} - (int64_t){self.cheap(x, z)}" + \
+                (" + 1)" if incl else ")")
+            out[d] = e if out[d] is None else f"ek::Min::op<int64_t>({out[d]}, {e})"
+        return out
+
+    def _clamped_load(self, op, lay: LY.Layout, V: int, nm: str, edge: list):
+        """A masked load at the edge of the selected box, without a branch per vector: every
+        vector is read, those that reach past the edge from the last V selected columns (and
+        the last selected row), so each address is one the mask selects; then the vectors that
+        moved are shifted back into place and filled with `other`. All loads of a thread are
+        in flight together, where one branch per vector made each wait for the one before it
+        (fp32 softmax, 4096 rows of 4101: 26.5 us with scalar loads, 28.3 us with a branch
+        per 16-byte vector). Needs V selected columns; a narrower box reads element by element."""
+        res, ptr = op.result, op.operands[0]
+        mask, other = op.operands[1], op.operands[2]
+        t = ctype(res.type.dtype)
+        rank, n = len(lay.shape), lay.nregs
+        dv, _ = lay.vec_dim_bits()
+        self.emit("{")
+        cs, room, eb = [], [], {}
+        for d in range(rank):
+            c = self.coord(lay, d, "rv")
+            if edge[d] is None:
+                cs.append(c)
+                continue
+            w = V if d == dv else 1
+            e = self.fresh("eb")
+            self.emit(f"  const int64_t {e}w = {edge[d]};")
+            self.emit(f"  const int {e} = (int)({e}w < {lay.shape[d]} ? ({e}w < 0 ? 0 : {e}w) : "
+                      f"{lay.shape[d]}) - {w};")
+            room.append(f"{e} >= 0")
+            eb[d] = f"{e} + {w}"
+            cs.append(f"ek::Min::op<int>({c}, {e})")
+        self.emit(f"  if ({' && '.join(room)}) {{")
+        self._vec_loop(n, V)
+        # a wave whose lanes all lie past the edge reads nothing
+        far = f"if (__builtin_amdgcn_ballot_w64({self.coord(lay, dv, 'rv')} < {eb[dv]})) " \
+            if edge[dv] is not None else ""
+        self.emit(f"    {far}ek::vload_u<{t}, {V}>(&{nm}[rv], {self.cheap(ptr, cs)});")
+        self.emit("  }")
+        self._vec_loop(n, V)
+        self.emit(f"    int ek_s = {self.coord(lay, dv, 'rv')} - {cs[dv]};"
+                  if edge[dv] is not None else "    int ek_s = 0;")
+        for d in range(rank):
+            if d != dv and edge[d] is not None:
+                self.emit(f"    if ({self.coord(lay, d, 'rv')} != {cs[d]}) ek_s = {V};")
+        self.emit("    if (__builtin_amdgcn_ballot_w64(ek_s != 0) != 0) {")
+        self.emit(f"      const {t} ek_o[{V}] = {{" + ", ".join(
+            self.elem(other, lay, f"rv + {i}" if i else "rv") for i in range(V)) + "};")
+        self.emit(f"      ek::edge_shift<{t}, {V}>(&{nm}[rv], ek_s, ek_o);")
+        self.emit("    }")
+        self.emit("  }")
+        self.emit("  } else {")
+        self.emit("  #pragma unroll")
+        self.emit(f"  for (int r = 0; r < {n}; ++r) {nm}[r] = ({self.elem(mask, lay, 'r')}) ? "
+                  f"*({self.elem(ptr, lay, 'r')}) : {self.elem(other, lay, 'r')};")
+        self.emit("  }")
+        self.emit("}")
 
     def _depends_on_pid(self, v: ir.Value, depth=0) -> bool:
         if v.op is None or depth > 48:
@@ -1413,7 +1554,8 @@ class Emitter:
         at = lambda i: f"{vals}[{base} + {i}]" if i else f"{vals}[{base}]"  # noqa: E731
         if own:
             self.emit(f"if ({own}) {{")
-        st = "vstore" if self.opt.get("no_nt_stores") else "vstore_nt"
+        st = ("vstore" if self.opt.get("no_nt_stores") else "vstore_nt") + \
+            self.vec_suffix(ptr, lay, V)
         cond = None
         if mask is not None and not self.opt.get("no_edge_versioning"):
             cond = self.all_true(mask)
@@ -1437,19 +1579,24 @@ class Emitter:
             self.emit("}")
             self.emit("} else {")
         self._vec_loop(lay.nregs, V)
-        open_vec()
         if mask is None:
+            open_vec()
             self.emit(f"  ek::{st}<{t}, {V}>({pe(0)}, &{at(0)});")
         else:
             me = lambda i: self.elem(mask, lay, f"rv + {i}" if i else "rv")  # noqa: E731
             if V > 1:
-                allm = " && ".join(f"({me(i)})" for i in range(V))
+                # a vector with no element selected is not computed either
+                allm, anym = self._vec_mask(mask, lay, V)
+                self.emit(f"  if ({anym}) {{")
+                open_vec()
                 self.emit(f"  if ({allm}) {{ ek::{st}<{t}, {V}>({pe(0)}, &{at(0)}); }}")
                 self.emit("  else {")
                 for i in range(V):
                     self.emit(f"    if ({me(i)}) *({pe(i)}) = {at(i)};")
                 self.emit("  }")
+                self.emit("  }")
             else:
+                open_vec()
                 self.emit(f"  if ({me(0)}) *({pe(0)}) = {at(0)};")
         self.emit("}")
         if cond:
@@ -1468,20 +1615,23 @@ class Emitter:
         self.desc[op.result.id] = info
         self.def_level[op.result.id] = len(self.scopes) - 1
 
-    def _desc_vec(self, d: dict, offs: list[ir.Value], lay: LY.Layout, es: int) -> int:
-        """Vector width for a descriptor block access in `lay` (contiguous last dim)."""
+    def _desc_vec(self, lay: LY.Layout, es: int) -> int:
+        """Vector width for a descriptor block access in `lay` (contiguous last dim, at any
+        alignment: see `mem_vec`)."""
         dvec, nb = lay.vec_dim_bits()
         rank = len(lay.shape)
         if dvec != rank - 1 or nb == 0:
             return 1
-        v = min(1 << nb, max(1, 16 // es))
+        return 1 << LY.log2(max(1, min(1 << nb, max(1, 16 // es))))
+
+    def _desc_suffix(self, d: dict, offs: list[ir.Value], V: int, es: int) -> str:
+        """`vec_suffix` for descriptor accesses of V elements."""
         align = self.axis.get(d["base_v"]).div[0]
         for o in offs[-1:]:
             align = math.gcd(align, self.axis.get(o).div[0] * es)
         for s in d["stride_v"][:-1]:
             align = math.gcd(align, self.axis.get(s).div[0] * es)
-        v = min(v, max(1, align // es))
-        return 1 << LY.log2(max(1, v))
+        return "" if V == 1 or align >= V * es else "_u"
 
     def _desc_addr(self, d, offs, lay, r):
         rank = len(lay.shape)
@@ -1503,7 +1653,8 @@ class Emitter:
         lay = self.lay[res.id]
         t = ctype(res.type.dtype)
         es = res.type.dtype.itemsize
-        V = self._desc_vec(d, offs, lay, es)
+        V = self._desc_vec(lay, es)
+        sfx = self._desc_suffix(d, offs, V, es)
         nm = self.fresh("dl")
         self.emit(f"{t} {nm}[{lay.nregs}];")
         self._vec_loop(lay.nregs, V)
@@ -1511,7 +1662,7 @@ class Emitter:
         zero = literal(0, res.type.dtype)
         if V > 1:
             _, cond_last = self._desc_addr(d, offs, lay, f"rv + {V - 1}")
-            self.emit(f"  if ({cond} && {cond_last}) {{ ek::vload<{t}, {V}>(&{nm}[rv], "
+            self.emit(f"  if ({cond} && {cond_last}) {{ ek::vload{sfx}<{t}, {V}>(&{nm}[rv], "
                       f"{d['base']} + {addr}); }}")
             self.emit("  else {")
             for i in range(V):
@@ -1530,13 +1681,14 @@ class Emitter:
         es = val.type.dtype.itemsize
         lay = LY.blocked(val.type.shape, LY.default_order(val.type.shape), max(1, 16 // es),
                          self.nw)
-        V = self._desc_vec(d, offs, lay, es)
+        V = self._desc_vec(lay, es)
+        sfx = self._desc_suffix(d, offs, V, es)
         vals = self.array(val, lay)
         self._vec_loop(lay.nregs, V)
         addr, cond = self._desc_addr(d, offs, lay, "rv")
         if V > 1:
             _, cond_last = self._desc_addr(d, offs, lay, f"rv + {V - 1}")
-            self.emit(f"  if ({cond} && {cond_last}) {{ ek::vstore_nt<{t}, {V}>({d['base']} + "
+            self.emit(f"  if ({cond} && {cond_last}) {{ ek::vstore_nt{sfx}<{t}, {V}>({d['base']} + "
                       f"{addr}, &{vals}[rv]); }}")
             self.emit("  else {")
             for i in range(V):

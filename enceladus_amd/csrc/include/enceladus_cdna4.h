@@ -224,6 +224,58 @@ template <typename T, int V> EK_INLINE void vstore(T* dst, const T* src) {
   *reinterpret_cast<R*>(dst) = v;
 }
 
+// The same moves at element alignment, for global memory: gfx950 runs vector loads and
+// stores at any alignment (the HSA queues' unaligned access mode, which hipcc's amdhsa
+// target assumes), so a row that starts at an odd element still moves 16 bytes per lane in
+// one instruction. Not for LDS, whose wide accesses need their alignment.
+template <typename T, int V> struct raw_u {
+  typedef typename raw_t<sizeof(T) * V>::type R;
+  typedef R type __attribute__((aligned(sizeof(T))));
+};
+template <typename T, int V> EK_INLINE void vload_u(T* dst, const T* src) {
+  const typename raw_u<T, V>::R v = *reinterpret_cast<const typename raw_u<T, V>::type*>(src);
+  __builtin_memcpy(dst, &v, sizeof(v));
+}
+template <typename T, int V> EK_INLINE void vload_nt_u(T* dst, const T* src) {
+  const typename raw_u<T, V>::R v =
+      __builtin_nontemporal_load(reinterpret_cast<const typename raw_u<T, V>::type*>(src));
+  __builtin_memcpy(dst, &v, sizeof(v));
+}
+template <typename T, int V> EK_INLINE void vstore_nt_u(T* dst, const T* src) {
+  typename raw_u<T, V>::R v;
+  __builtin_memcpy(&v, src, sizeof(v));
+  __builtin_nontemporal_store(v, reinterpret_cast<typename raw_u<T, V>::type*>(dst));
+}
+template <typename T, int V> EK_INLINE void vstore_u(T* dst, const T* src) {
+  typename raw_u<T, V>::R v;
+  __builtin_memcpy(&v, src, sizeof(v));
+  *reinterpret_cast<typename raw_u<T, V>::type*>(dst) = v;
+}
+
+// A vector read `s` elements early (s >= V: not selected at all), put back in place: element
+// i is v[i + s], or o[i] past the vector's end. The vector is shifted as one integer, which
+// keeps it in registers whatever `s` is.
+template <int N> struct bits_of { typedef unsigned __int128 type; };
+template <> struct bits_of<2> { typedef uint16_t type; };
+template <> struct bits_of<4> { typedef uint32_t type; };
+template <> struct bits_of<8> { typedef uint64_t type; };
+template <typename T, int V> EK_INLINE void edge_shift(T* v, int s, const T* o) {
+  typedef typename bits_of<sizeof(T) * V>::type U;
+  static_assert(sizeof(U) == sizeof(T) * V, "vectors of 2 to 16 bytes");
+  constexpr int B = sizeof(T) * 8;
+  if (__builtin_amdgcn_ballot_w64(s > 0 && s < V) != 0) {
+    U x, f;
+    __builtin_memcpy(&x, v, sizeof(U));
+    __builtin_memcpy(&f, o, sizeof(U));
+    const int n = B * (s & (V - 1));
+    const U sel = (U)(~(U)0 >> n);            // the V - s elements that were read
+    x = (U)((x >> n) & sel) | (U)(f & (U)~sel);
+    __builtin_memcpy(v, &x, sizeof(U));
+  }
+#pragma unroll
+  for (int i = 0; i < V; ++i) v[i] = s >= V ? o[i] : v[i];
+}
+
 // ---------------------------------------------------------------------------
 // Wave64 cross-lane moves.
 // ---------------------------------------------------------------------------
