@@ -960,11 +960,15 @@ class Emitter:
         t = ctype(src.type.dtype) + ("*" if src.type.ptr else "")
         es = 8 if src.type.ptr else src.type.dtype.itemsize
         order = self.lds_order(a, dst, es)
-        strides, total = self.lds_addr(a.shape, order, es)
+        # a tile larger than the LDS moves in 2^k passes, each the part whose coordinate along
+        # the image's slowest dim has the pass number in its top bits
+        shape, k = list(a.shape), 0
+        strides, total = self.lds_addr(shape, order, es)
+        while total * es > MAX_LDS:
+            shape[order[-1]] //= 2
+            k += 1
+            strides, total = self.lds_addr(shape, order, es)
         nbytes = total * es
-        if nbytes > MAX_LDS:
-            raise CompilationError(f"a layout conversion of a {a.shape} tile needs {nbytes} "
-                                   "bytes of LDS")
         self.need_lds(nbytes)
         op = getattr(self, "cur_op", None)
         self.report.setdefault("conversions", []).append(
@@ -976,17 +980,30 @@ class Emitter:
         wv = self.lds_vec(a, order, es)
         rv = self.lds_vec(dst, order, es)
         lines.append(f"{t} {nm}[{dst.nregs}];")
-        lines.append("{")
-        lines.append(f"  {t}* sm = reinterpret_cast<{t}*>(ek_smem);")
-        lines.append("  __syncthreads();")
-        lines.append("  #pragma unroll")
-        lines.append(f"  for (int r = 0; r < {a.nregs}; r += {wv}) "
-                     f"ek::vstore<{t}, {wv}>(&sm[{self.lds_index(a, strides, 'r')}], &{sname}[r]);")
-        lines.append("  __syncthreads();")
-        lines.append("  #pragma unroll")
-        lines.append(f"  for (int r = 0; r < {dst.nregs}; r += {rv}) "
-                     f"ek::vload<{t}, {rv}>(&{nm}[r], &sm[{self.lds_index(dst, strides, 'r')}]);")
-        lines.append("}")
+        for p in range(1 << k):
+            def part(lay):
+                """(condition, index) of register `r` of `lay` in this pass."""
+                ix = self.lds_index(lay, strides, "r")
+                if not k:
+                    return "", ix
+                d = order[-1]
+                c = self.coord(lay, d, "r")
+                if p:
+                    ix = f"({ix}) - {p * shape[d] * strides[d]}"
+                return f"if ((({c}) >> {LY.log2(shape[d])}) == {p}) ", ix
+            lines.append("{")
+            lines.append(f"  {t}* sm = reinterpret_cast<{t}*>(ek_smem);")
+            lines.append("  __syncthreads();")
+            lines.append("  #pragma unroll")
+            cond, ix = part(a)
+            lines.append(f"  for (int r = 0; r < {a.nregs}; r += {wv}) {cond}"
+                         f"ek::vstore<{t}, {wv}>(&sm[{ix}], &{sname}[r]);")
+            lines.append("  __syncthreads();")
+            lines.append("  #pragma unroll")
+            cond, ix = part(dst)
+            lines.append(f"  for (int r = 0; r < {dst.nregs}; r += {rv}) {cond}"
+                         f"ek::vload<{t}, {rv}>(&{nm}[r], &sm[{ix}]);")
+            lines.append("}")
         self._emit_at_level(lvl, lines)
         self.scopes[lvl].memo[key] = nm
         return nm
@@ -1532,6 +1549,12 @@ class Emitter:
             if vl.shape == lay.shape and (self.mem_vec(ptr, vl) >= want or
                                           self.wave_run_bytes(ptr, vl) >= 256):
                 lay = vl
+        if self.kind.get(val.id) == "fused" and self.lay[val.id].key() != lay.key():
+            # the stored value moves to another layout: it is computed where its operands are
+            # and moved in its own type (a matmul's result as 16 bits, not as its accumulator)
+            nm = self.array(val, self.lay[val.id])
+            self.kind[val.id] = "anchored"
+            self.define(val, nm)
         V = self.mem_vec(ptr, lay)
         own = self.owner_cond(lay)
         self.prime((ptr, lay), (mask, lay), (val, lay))

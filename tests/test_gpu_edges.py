@@ -69,3 +69,22 @@ def test_box_edges(shape, dtype):
     want = torch.full_like(tile.cpu(), -3.0)
     want[:rows, :cols] = x.cpu()[:, :cols]
     assert torch.equal(tile.cpu(), want)
+
+
+@enceladus.jit
+def _transpose(x_ptr, o_ptr, M: tl.constexpr, N: tl.constexpr):
+    r, c = tl.arange(0, M), tl.arange(0, N)
+    x = tl.load(x_ptr + r[:, None] * N + c[None, :])
+    tl.store(o_ptr + c[:, None] * M + r[None, :], tl.trans(x))
+
+
+@pytest.mark.parametrize("shape", [(128, 256), (256, 256), (512, 128), (16, 4096)])
+@pytest.mark.parametrize("dtype", ["float32", "float16", "int64"])
+def test_layout_conversions_larger_than_the_lds(shape, dtype):
+    """256 x 256 float32 tiles (256 KB) and wider ones move through LDS in passes."""
+    import torch
+    m, n = shape
+    x = torch.arange(m * n, device="cuda").remainder(2039).to(getattr(torch, dtype)).view(m, n)
+    o = torch.zeros(n, m, dtype=x.dtype, device="cuda")
+    _transpose[(1,)](x, o, M=m, N=n, num_warps=8)
+    assert torch.equal(o, x.t())
