@@ -78,7 +78,9 @@ class AxisAnalysis:
             body = op.regions[0]
             carried = body.args[1:]
             inits = op.operands[3:]
-            self.info[body.args[0].id] = _scalar(1)
+            # lo, lo + step, lo + 2 * step, ...
+            self.info[body.args[0].id] = _scalar(math.gcd(self.get(op.operands[0]).div[0],
+                                                          self.get(op.operands[2]).div[0]))
             for a, i in zip(carried, inits):
                 self.info[a.id] = self.get(i)
             for _ in range(3):
@@ -170,6 +172,10 @@ class AxisAnalysis:
             elif kind == "sub":
                 contig = tuple(math.gcd(ca, kb) for ca, kb in zip(a.contig, b.const))
                 div = tuple(math.gcd(x, y) for x, y in zip(a.div, b.div))
+            elif kind in ("min", "max"):
+                # whichever is picked, a common divisor of both divides it
+                contig = (1,) * rank
+                div = tuple(math.gcd(x, y) for x, y in zip(a.div, b.div))
             elif kind == "mul":
                 contig = (1,) * rank
                 div = tuple(min(x * y, BIG) for x, y in zip(a.div, b.div))
@@ -183,6 +189,11 @@ class AxisAnalysis:
             if res.type.dtype.is_int() and op.operands[0].type.dtype.is_int() and \
                     res.type.dtype.primitive_bitwidth >= op.operands[0].type.dtype.primitive_bitwidth:
                 self.info[res.id] = s
+            elif res.type.dtype.is_int() and op.operands[0].type.dtype.is_int() and \
+                    not res.type.dtype.is_bool():
+                # a narrowing cast drops high bits: powers of two below them still divide
+                top = 1 << (res.type.dtype.primitive_bitwidth - 1)
+                self.info[res.id] = Info((1,) * rank, tuple(min(d, top) for d in s.div), s.const)
             else:
                 self.info[res.id] = Info((1,) * rank, (1,) * rank, s.const)
         elif n in ("unary", "bitcast"):

@@ -3298,15 +3298,11 @@ class Emitter:
             return None
         nt = self.nt
         kc = bk // 8
-        if bk % 16 or (bm * kc) % nt or ((kc * (bn // 8)) % nt and kc * (bn // 8) >= nt):
+        if bk % 16:
             return None
         if self.lay[acc.id].key() != LY.mfma_acc(plan).key():
             return None
         A, B = self.desc[da.id], self.desc[db.id]
-        ok = lambda v, d: self.axis.get(v).div[0] >= d  # noqa: E731
-        if not (ok(A["base_v"], 16) and ok(B["base_v"], 16) and ok(A["stride_v"][0], 8)
-                and ok(B["stride_v"][0], 8)):
-            return None
         return {"plan": plan, "A": A, "B": B, "m0": la.operands[1], "n0": lb.operands[2],
                 "scalar_ops": scalar_ops, "dt": dt, "bm": bm, "bn": bn, "bk": bk}
 
@@ -3328,11 +3324,14 @@ class Emitter:
         p = g["plan"]
         T = ctype(g["dt"])
         A, B = g["A"], g["B"]
-        # Buffer loads (hardware bounds checks) send a 16-byte chunk that is not wholly inside
-        # its row out of range, so they need K and N known to be multiples of 8; and no
-        # operand may span >= 2 GiB (32-bit byte offsets).
+        # LDS DMA needs rows of whole 16-byte chunks (bases, strides, K and N known to be
+        # multiples of 8 elements: a chunk is then wholly inside its row or out of range) and
+        # 32-bit byte offsets; anything else goes through registers (ek::GemmReg).
+        div = lambda v: self.axis.get(v).div[0]  # noqa: E731
         big = any(v.facts.get("span2g") for v in (A["base_v"], B["base_v"]))
-        whole = all(self.axis.get(v).div[0] % 8 == 0 for v in (A["shape_v"][1], B["shape_v"][1]))
+        rows = all(div(v) >= 16 for v in (A["base_v"], B["base_v"])) and \
+            all(div(v) % 8 == 0 for v in (A["stride_v"][0], B["stride_v"][0]))
+        whole = rows and all(div(v) % 8 == 0 for v in (A["shape_v"][1], B["shape_v"][1]))
         buf = not (big or not whole or self.opt.get("no_buffer_loads"))
         bm, bn, bk = g["bm"], g["bn"], g["bk"]
         stage = (bm * bk + bk * bn) * 2
@@ -3352,9 +3351,8 @@ class Emitter:
                     f"{split}{tr}>")
             self.need_lds(nst * stage)
         else:
-            tr = ", true" if p.trans else ""
-            tmpl = (f"ek::Gemm<{T}, {bm}, {bn}, {bk}, {p.wm}, {p.wn}, {self.nt}, "
-                    f"{'true' if buf else 'false'}{tr}>")
+            tmpl = (f"ek::{'Gemm' if rows else 'GemmReg'}<{T}, {bm}, {bn}, {bk}, {p.wm}, {p.wn}, "
+                    f"{self.nt}, {'true' if big else 'false'}{', true' if p.trans else ''}>")
             self.need_lds(2 * stage)
         self.emit(f"  {tmpl} ek_g;")
         self.emit(f"  ek_g.run({nm}, {A['base']}, {A['strides'][0]}, {B['base']}, "

@@ -505,24 +505,6 @@ EK_INLINE void mfma_16x16x32(int32_t* acc, const int8_t* a, const int8_t* b) {
 }
 
 
-// ---------------------------------------------------------------------------
-// Block GEMM main loop for `for k in range(lo, hi, BK): acc = dot(A.load([m0, k]),
-// B.load([k, n0]), acc)` with row-major 16-bit A [M, K] (lda) and B [K, N] (ldb).
-//
-// NT threads = WM x WN waves; each wave owns a (BM/WM) x (BN/WN) block of 32x32 MFMA tiles
-// (v_mfma_f32_32x32x16_{f16,bf16}). The accumulator is held in the emitter's MFMA layout:
-// acc[(tm * TN + tn) * 16 + j]. With TR the instruction computes each tile's transpose
-// (B^T A^T, the same fragments in swapped slots), so a lane holds one row of C and 4
-// consecutive columns per 4 registers instead of one column and 4 rows.
-//
-// Per iteration each thread prefetches its share of the next A and B tiles from global
-// memory into registers (16-byte loads), computes the current tile from LDS, then writes
-// the prefetched registers into the other LDS stage: one barrier per iteration.
-// LDS holds A as [BM][BK] and B transposed as [BN][BK], both with k contiguous and the
-// 16-byte chunk index XOR-swizzled by the row, so every MFMA operand is one 128-bit LDS
-// read. B is transposed in registers: each thread loads an 8x8 block (8 k rows x 8 n
-// columns) and permutes it with v_perm_b32 before writing 8 rows of B^T.
-// ---------------------------------------------------------------------------
 EK_INLINE uint32_t perm_lo(uint32_t lo_src, uint32_t hi_src) {
   return __builtin_amdgcn_perm(hi_src, lo_src, 0x05040100u);  // (lo16(lo_src), lo16(hi_src))
 }
@@ -682,172 +664,246 @@ EK_INLINE void dma16(i32x4 rsrc, uint32_t lds, int voff) {
                ::"s"(lds), "v"(voff), "s"(rsrc) : "memory", "m0");
 }
 
-template <typename T, int BM, int BN, int BK, int WM, int WN, int NT, bool BUF = false,
-          bool TR = false>
-struct Gemm {
+// ---------------------------------------------------------------------------
+// Block GEMM loops for `for k in range(lo, hi, BK): acc = dot(A.load([m0, k]),
+// B.load([k, n0]), acc)` with row-major 16-bit A [M, K] (lda) and B [K, N] (ldb).
+//
+// NT threads = WM x WN waves; each wave owns a (BM/WM) x (BN/WN) block of 32x32 MFMA tiles
+// (v_mfma_f32_32x32x16_{f16,bf16}). The accumulator is held in the emitter's MFMA layout:
+// acc[(tm * TN + tn) * 16 + j]. With TR the instruction computes each tile's transpose
+// (B^T A^T, the same fragments in swapped slots), so a lane holds one row of C and 4
+// consecutive columns per 4 registers instead of one column and 4 rows.
+//
+// GemmTile is one stage in LDS and the MFMAs on it: A [BM][BK] and B [BK][BN] row-major in
+// 16-byte chunks. A fragments are 16-byte reads; B's k-major fragments come from
+// ds_read_b64_tr_b16: in each group of 16 lanes, lane 4i + q reads 4 columns of k row i, and
+// output lane L receives column L of the 4 rows. LDS swizzles (reads are served 256 bytes per
+// pass): A chunk (row, kc) sits at row * KC + (kc ^ ((row >> ASH) & AMASK)); B chunk (k, nc)
+// at k * NCB + (nc ^ (((k >> RSH) & RMASK) << 2)), which spreads the 4 rows a transpose read
+// touches over the 4 64-byte quarters of a pass.
+// ---------------------------------------------------------------------------
+template <typename T, int BM, int BN, int BK, int WM, int WN, int NT, bool TR>
+struct GemmTile {
   static constexpr int TM = BM / WM / 32, TN = BN / WN / 32, TK = BK / 16;
-  static constexpr int KC = BK / 8;                    // 16-byte chunks per k row
-  static constexpr int A_CH = BM * KC / NT;            // A chunks per thread
-  static constexpr int B_TOTAL = KC * (BN / 8);        // B 8x8 blocks per tile
-  static constexpr int B_BL = (B_TOTAL + NT - 1) / NT; // B 8x8 blocks per thread
-  static constexpr int STAGE = (BM + BN) * BK;         // elements per LDS stage
-  static constexpr int LDS_BYTES = 2 * STAGE * 2;
-  static_assert(TM >= 1 && TN >= 1 && TK >= 1, "tile too small for 32x32x16 MFMA");
-  static_assert((BM * KC) % NT == 0 && (B_TOTAL % NT == 0 || B_TOTAL < NT),
-                "tile/thread mismatch");
-  static_assert(WM * WN * 64 == NT, "warps must tile the block");
-
-  u32x4 ra[A_CH];
-  u32x4 rb[B_BL][8];
-
-  EK_INLINE void load(const uint16_t* A, int lda, const uint16_t* B, int ldb, int M, int N,
-                      int K, int m0, int n0, int k, int tid) {
-    if constexpr (BUF) {
-      // Rows past M (A) or K (B) fall outside the resources; chunks past the last column
-      // are sent out of range explicitly.
-      const __amdgpu_buffer_rsrc_t ra_r = buffer_rsrc(A, (uint32_t)M * lda * 2);
-      const __amdgpu_buffer_rsrc_t rb_r = buffer_rsrc(B, (uint32_t)K * ldb * 2);
-#pragma unroll
-      for (int i = 0; i < A_CH; ++i) {
-        const int c = tid + i * NT, row = c / KC, kc = c % KC;
-        const int gk = k + kc * 8;
-        const int off = (gk + 8 <= K) ? ((m0 + row) * lda + gk) * 2 : kOOB;
-        ra[i] = buffer_load16(ra_r, off);
-      }
-#pragma unroll
-      for (int i = 0; i < B_BL; ++i) {
-        const int b = tid + i * NT, nb = b % (BN / 8), kb = b / (BN / 8);
-        if (B_TOTAL < NT && b >= B_TOTAL) break;
-        const int gn = n0 + nb * 8;
-        const int base = (gn + 8 <= N) ? ((k + kb * 8) * ldb + gn) * 2 : kOOB;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          rb[i][j] = buffer_load16(rb_r, base == kOOB ? kOOB : base + j * ldb * 2);
-      }
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < A_CH; ++i) {
-      const int c = tid + i * NT, row = c / KC, kc = c % KC;
-      const int gr = m0 + row, gk = k + kc * 8;
-      if ((unsigned)gr < (unsigned)M && gk >= 0 && gk + 8 <= K) {
-        ra[i] = *reinterpret_cast<const u32x4*>(A + (int64_t)gr * lda + gk);
-      } else {
-        uint16_t h[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          h[e] = ((unsigned)gr < (unsigned)M && (unsigned)(gk + e) < (unsigned)K)
-                     ? A[(int64_t)gr * lda + gk + e] : 0;
-        __builtin_memcpy(&ra[i], h, 16);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < B_BL; ++i) {
-      const int b = tid + i * NT, nb = b % (BN / 8), kb = b / (BN / 8);
-      if (B_TOTAL < NT && b >= B_TOTAL) break;
-      const int gn = n0 + nb * 8;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int gk = k + kb * 8 + j;
-        if ((unsigned)gk < (unsigned)K && gn >= 0 && gn + 8 <= N) {
-          rb[i][j] = *reinterpret_cast<const u32x4*>(B + (int64_t)gk * ldb + gn);
-        } else {
-          uint16_t h[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            h[e] = ((unsigned)gk < (unsigned)K && (unsigned)(gn + e) < (unsigned)N)
-                       ? B[(int64_t)gk * ldb + gn + e] : 0;
-          __builtin_memcpy(&rb[i][j], h, 16);
-        }
-      }
-    }
-  }
-
-  // LDS addressing (in 16-byte chunks). gfx950 serves LDS reads 256 bytes per pass (16
-  // lanes of 16 bytes) and writes 128 bytes per pass (8 lanes). A: row-major [BM][KC]
-  // chunks, chunk index xor'ed with (row >> ASH) & AMASK, so the 16 rows a read pass
-  // touches land on 16 distinct chunk slots and a write pass (8 chunks of one row) stays
-  // contiguous. B^T: k-chunk-major [KC][BN] chunks with the column permuted as
-  // n ^ ((n >> 3) & 7), so reads of 16 consecutive columns and writes of the 8 columns
-  // n = 8 nb + q (one per 8x8 block) are both conflict-free.
+  static constexpr int KC = BK / 8;                       // A chunks per row
+  static constexpr int NCB = BN / 8;                      // B chunks per row
+  static constexpr int A_ELEMS = BM * BK, STAGE = BM * BK + BK * BN;
   static constexpr int ASH = KC >= 16 ? 0 : (KC == 8 ? 1 : (KC == 4 ? 2 : 3));
   static constexpr int AMASK = (KC < 16 ? KC : 16) - 1;
-  static EK_INLINE int a_chunk(int row, int kc) { return row * KC + (kc ^ ((row >> ASH) & AMASK)); }
-  static EK_INLINE int b_chunk(int n, int kc) { return kc * BN + (n ^ ((n >> 3) & 7)); }
+  static constexpr int RP = BN >= 128 ? 1 : 128 / BN;     // B rows per 256 bytes
+  static constexpr int RSH = RP == 1 ? 0 : (RP == 2 ? 1 : 2);
+  static constexpr int RMASK = 4 / RP - 1;
+  static_assert(TM >= 1 && TN >= 1 && TK >= 1, "tile too small for 32x32x16 MFMA");
+  static_assert(WM * WN * 64 == NT, "warps must tile the block");
+  static_assert(NCB >= 4 * (RMASK + 1), "B swizzle needs the row's chunks");
 
-  EK_INLINE void store(uint16_t* st, int tid) {
-    u32x4* sA = reinterpret_cast<u32x4*>(st);
-    u32x4* sB = reinterpret_cast<u32x4*>(st + BM * BK);
+  static EK_INLINE int a_chunk(int row, int kc) { return row * KC + (kc ^ ((row >> ASH) & AMASK)); }
+  static EK_INLINE int b_chunk(int k, int nc) { return k * NCB + (nc ^ (((k >> RSH) & RMASK) << 2)); }
+
+  // One k slice: every A and B fragment read, then the TM x TN MFMAs.
+  EK_INLINE void compute_kk(int kk, float* acc, const uint16_t* st, int lane, int wm, int wn) {
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    const u32x4* sA = reinterpret_cast<const u32x4*>(st);
+    const uint16_t* sB = st + A_ELEMS;
+    const int r32 = lane & 31, h = lane >> 5;
+    const int g = lane >> 4, ti = (lane >> 2) & 3, tq = lane & 3;
+    T a[TM][8], b[TN][8];
+    const int kc = kk * 2 + h;
 #pragma unroll
-    for (int i = 0; i < A_CH; ++i) {
-      const int c = tid + i * NT, row = c / KC, kc = c % KC;
-      sA[a_chunk(row, kc)] = ra[i];
+    for (int tm = 0; tm < TM; ++tm) {
+      const u32x4 v = sA[a_chunk(wm * (BM / WM) + tm * 32 + r32, kc)];
+      __builtin_memcpy(a[tm], &v, 16);
     }
 #pragma unroll
-    for (int i = 0; i < B_BL; ++i) {
-      const int b = tid + i * NT, nb = b % (BN / 8), kb = b / (BN / 8);
-      if (B_TOTAL < NT && b >= B_TOTAL) break;
-      u32x4 o[8];
-      transpose8x8(rb[i], o);
+    for (int tn = 0; tn < TN; ++tn) {
+      const int n = wn * (BN / WN) + tn * 32 + 16 * (g & 1) + 4 * tq;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) sB[b_chunk(nb * 8 + q, kb)] = o[q];
+      for (int half = 0; half < 2; ++half) {
+        const int k = kk * 16 + 8 * (g >> 1) + 4 * half + ti;
+        const uint16_t* src = sB + b_chunk(k, n >> 3) * 8 + (n & 7);
+        const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4s*)(src));
+        __builtin_memcpy(&b[tn][4 * half], &v, 8);
+      }
+    }
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) {
+        if constexpr (TR) mfma_32x32x16(&acc[(tm * TN + tn) * 16], b[tn], a[tm]);
+        else mfma_32x32x16(&acc[(tm * TN + tn) * 16], a[tm], b[tn]);
+      }
+  }
+
+  template <int KK0, int KK1>
+  EK_INLINE void compute(float* acc, const uint16_t* st, int lane, int wm, int wn) {
+#pragma unroll
+    for (int kk = KK0; kk < KK1; ++kk) compute_kk(kk, acc, st, lane, wm, wn);
+  }
+};
+
+// ---------------------------------------------------------------------------
+// The loop for operands of any alignment and size, through registers: each thread loads its
+// 16-byte chunks of the tile PD steps ahead (element-aligned vector loads) and writes the tile
+// that has arrived to the other of two LDS stages, one barrier per step.
+//
+// What bounds it: with rows at odd element offsets there is no LDS DMA and no aligned chunk,
+// so the loads' latency has to be covered from registers (PD steps of them) and each byte
+// crosses the VGPRs. Edges cost no per-element loads: a chunk past the last row or column is
+// read from the last row, or from the row's last 8 columns and shifted into place, so every
+// address lies inside the operand; offsets are fixed before the loop (one set for the last k
+// step, which may be ragged). Operands narrower than a chunk, and tiles that start before the
+// operand, are read element by element.
+// ---------------------------------------------------------------------------
+template <typename T, int BM, int BN, int BK, int WM, int WN, int NT, bool BIG, bool TR = false>
+struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
+  typedef GemmTile<T, BM, BN, BK, WM, WN, NT, TR> G;
+  using G::TK, G::KC, G::NCB, G::A_ELEMS, G::STAGE;
+  static constexpr int A_TOT = BM * KC, B_TOT = BK * NCB;
+  static constexpr int A_CH = (A_TOT + NT - 1) / NT, B_CH = (B_TOT + NT - 1) / NT;
+  static constexpr int CH = A_CH + B_CH;
+  // k steps of loads in flight: about 32 registers' worth (64x64x32 tiles on 4 waves, bf16
+  // 1000 x 3000 x 2000: 35.6 us at 4 steps, 38.9 at 1; 256x256x64 on 8 waves spills at 2)
+  static constexpr int PD = CH <= 2 ? 4 : CH <= 4 ? 2 : 1;
+  static constexpr int LDS_BYTES = 2 * STAGE * 2;
+  // byte offsets from a tile's k origin: 32 bits, or 64 for operands of 2 GiB and more
+  template <bool> struct off_of { typedef uint32_t type; };
+  template <> struct off_of<true> { typedef int64_t type; };
+  typedef typename off_of<BIG>::type Off;
+  typedef u32x4 chunk __attribute__((aligned(2)));
+
+  u32x4 r[PD][CH];
+  // Of each chunk, from a k step's first column less 8 (A: a chunk moved back from a ragged
+  // end starts up to 7 columns before it) or first row (B).
+  Off off[CH], last[CH];    // of every k step, and of the last one
+  int sh[CH], lsh[CH];      // elements to shift (8 and more: all zero), likewise
+
+  static EK_INLINE int row_a(int i, int tid) { return (i * NT + tid) / KC; }
+  static EK_INLINE int kc_a(int i, int tid) { return (i * NT + tid) % KC; }
+  static EK_INLINE int row_b(int i, int tid) { return (i * NT + tid) / NCB; }
+  static EK_INLINE int nc_b(int i, int tid) { return (i * NT + tid) % NCB; }
+  // whether chunk i exists for this thread (always, when the tile fills the threads evenly)
+  static EK_INLINE bool has(int i, int tid) {
+    if (i < A_CH) return A_TOT % NT == 0 || i * NT + tid < A_TOT;
+    return B_TOT % NT == 0 || (i - A_CH) * NT + tid < B_TOT;
+  }
+
+  EK_INLINE void plan(int lda, int ldb, int M, int N, int K, int m0, int n0, int klast, int tid) {
+#pragma unroll
+    for (int i = 0; i < A_CH; ++i) {
+      const int row = m0 + row_a(i, tid), rc = Min::op<int>(row, M - 1), c = kc_a(i, tid) * 8;
+      const int cl = Min::op<int>(klast + c, K - 8) - klast;     // -7 and more
+      off[i] = ((Off)rc * (Off)lda + (Off)(c + 8)) * 2;
+      last[i] = ((Off)rc * (Off)lda + (Off)(cl + 8)) * 2;
+      sh[i] = row < M ? 0 : 8;
+      lsh[i] = row < M ? c - cl : 8;
+    }
+#pragma unroll
+    for (int j = 0; j < B_CH; ++j) {
+      const int i = A_CH + j, k = row_b(j, tid), gn = n0 + nc_b(j, tid) * 8;
+      const int kl = Min::op<int>(klast + k, K - 1) - klast, nl = Min::op<int>(gn, N - 8);
+      off[i] = ((Off)k * (Off)ldb + (Off)nl) * 2;
+      last[i] = ((Off)kl * (Off)ldb + (Off)nl) * 2;
+      sh[i] = gn - nl;
+      lsh[i] = kl == k ? gn - nl : 8;
     }
   }
 
-  EK_INLINE void compute(float* acc, const uint16_t* st, int lane, int wm, int wn) {
-    const u32x4* sA = reinterpret_cast<const u32x4*>(st);
-    const u32x4* sB = reinterpret_cast<const u32x4*>(st + BM * BK);
-    const int r32 = lane & 31, h = lane >> 5;
+  EK_INLINE void load(int p, const char* a, const char* b, bool end, int tid) {
 #pragma unroll
-    for (int kk = 0; kk < TK; ++kk) {
-      T a[TM][8], b[TN][8];
-      const int kc = kk * 2 + h;
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm) {
-        const u32x4 v = sA[a_chunk(wm * (BM / WM) + tm * 32 + r32, kc)];
-        __builtin_memcpy(a[tm], &v, 16);
-      }
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) {
-        const u32x4 v = sB[b_chunk(wn * (BN / WN) + tn * 32 + r32, kc)];
-        __builtin_memcpy(b[tn], &v, 16);
-      }
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) {
-          if constexpr (TR) mfma_32x32x16(&acc[(tm * TN + tn) * 16], b[tn], a[tm]);
-          else mfma_32x32x16(&acc[(tm * TN + tn) * 16], a[tm], b[tn]);
-        }
+    for (int i = 0; i < CH; ++i) {
+      const char* q = (i < A_CH ? a : b) + (end ? last[i] : off[i]);
+      if (has(i, tid)) r[p][i] = *reinterpret_cast<const chunk*>(q);
     }
+  }
+
+  EK_INLINE void put(int p, uint16_t* st, int tid) {
+    u32x4* sA = reinterpret_cast<u32x4*>(st);
+    u32x4* sB = reinterpret_cast<u32x4*>(st + A_ELEMS);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      if (!has(i, tid)) continue;
+      if (i < A_CH) sA[G::a_chunk(row_a(i, tid), kc_a(i, tid))] = r[p][i];
+      else sB[G::b_chunk(row_b(i - A_CH, tid), nc_b(i - A_CH, tid))] = r[p][i];
+    }
+  }
+
+  EK_INLINE void shift(int p, bool end) {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int s = end ? lsh[i] : sh[i];
+      unsigned __int128 x = __builtin_bit_cast(unsigned __int128, r[p][i]);
+      x = s >= 8 ? 0 : x >> (16 * (s & 7));
+      r[p][i] = __builtin_bit_cast(u32x4, x);
+    }
+  }
+
+  // One element of an operand [rows, cols], zero outside it.
+  static EK_INLINE uint16_t at(const T* P, int64_t ld, int rows, int cols, int i, int j) {
+    if (i < 0 || i >= rows || j < 0 || j >= cols) return 0;
+    return reinterpret_cast<const uint16_t*>(P)[i * ld + j];
   }
 
   // Runs the whole k loop: k = lo, lo + BK, ... < hi.
   EK_INLINE void run(float* acc, const T* A, int lda, const T* B, int ldb, int M, int N, int K,
                      int m0, int n0, int lo, int hi, char* smem, int tid) {
+    hi = Min::op<int>(hi, K);   // past K both operands are zero
     if (hi <= lo) return;
-    const int niter = (hi - lo + BK - 1) / BK;
+    const int niter = (int)(((int64_t)hi - lo + BK - 1) / BK);
     const int lane = tid & 63, warp = tid >> 6;
     const int wm = warp % WM, wn = warp / WM;
-    const uint16_t* A16 = reinterpret_cast<const uint16_t*>(A);
-    const uint16_t* B16 = reinterpret_cast<const uint16_t*>(B);
     uint16_t* s16 = reinterpret_cast<uint16_t*>(smem);
-    __syncthreads();
-    load(A16, lda, B16, ldb, M, N, K, m0, n0, lo, tid);
-    store(s16, tid);
-    __syncthreads();
-    // s_waitcnt vmcnt(0): nothing loaded before the loop (the accumulator's initial value
-    // included) is outstanding at its head, so the first MFMA does not wait for the prefetch.
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    for (int it = 0; it < niter; ++it) {
-      const bool more = it + 1 < niter;
-      if (more) load(A16, lda, B16, ldb, M, N, K, m0, n0, lo + (it + 1) * BK, tid);
-      compute(acc, s16 + (it & 1) * STAGE, lane, wm, wn);
-      if (more) store(s16 + ((it + 1) & 1) * STAGE, tid);
-      __syncthreads();
+    __syncthreads();  // earlier users of the LDS are done with it
+    if (m0 < 0 || n0 < 0 || lo < 0 || M < 1 || N < 8 || K < 8) {
+      for (int it = 0; it < niter; ++it) {
+        const int k = lo + it * BK;
+        for (int c = tid; c < BM * BK; c += NT)
+          s16[G::a_chunk(c / BK, (c % BK) / 8) * 8 + c % 8] =
+              at(A, lda, M, K, m0 + c / BK, k + c % BK);
+        for (int c = tid; c < BK * BN; c += NT)
+          s16[A_ELEMS + G::b_chunk(c / BN, (c % BN) / 8) * 8 + c % 8] =
+              at(B, ldb, K, N, k + c / BN, n0 + c % BN);
+        __syncthreads();
+        G::template compute<0, TK>(acc, s16, lane, wm, wn);
+        __syncthreads();
+      }
+      return;
     }
+    const int klast = lo + (niter - 1) * BK;
+    const bool edge = m0 + BM > M || n0 + BN > N, ragged = klast + BK > K;
+    plan(lda, ldb, M, N, K, m0, n0, klast, tid);
+    const char* a = reinterpret_cast<const char*>(A) + ((int64_t)lo - 8) * 2;
+    const char* b = reinterpret_cast<const char*>(B) + (int64_t)lo * ldb * 2;
+    const int64_t sa = BK * 2, sb = (int64_t)BK * ldb * 2;
+#pragma unroll
+    for (int p = 0; p < PD; ++p) {
+      const int t = Min::op<int>(p, niter - 1);
+      load(p, a + t * sa, b + t * sb, t == niter - 1, tid);
+    }
+    for (int it = 0; it < niter; it += PD) {
+#pragma unroll
+      for (int p = 0; p < PD; ++p) {
+        const int t = it + p;
+        if (t >= niter) break;
+        const bool end = t == niter - 1;
+        if (edge || (end && ragged)) shift(p, end);
+        uint16_t* st = s16 + (PD % 2 ? (t & 1) : (p & 1)) * STAGE;
+        put(p, st, tid);
+        // past the end: the last tile again, which nothing reads
+        const int nx = Min::op<int>(t + PD, niter - 1);
+        load(p, a + nx * sa, b + nx * sb, nx == niter - 1, tid);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        G::template compute<0, TK>(acc, st, lane, wm, wn);
+      }
+    }
+    __syncthreads();
   }
 };
+
+// Operands whose rows are known to start on 16 bytes (K or N are not whole chunks): only the
+// chunks moved at an edge are unaligned.
+template <typename T, int BM, int BN, int BK, int WM, int WN, int NT, bool BIG, bool TR = false>
+using Gemm = GemmReg<T, BM, BN, BK, WM, WN, NT, BIG, TR>;
 
 // ---------------------------------------------------------------------------
 // GEMM main loop fed by LDS DMA: C[BM x BN] += A[BM x K] * B[K x BN], 16-bit row-major
@@ -871,29 +927,16 @@ struct Gemm {
 // ---------------------------------------------------------------------------
 template <typename T, int BM, int BN, int BK, int WM, int WN, int NT, int S, int SPLIT = 1,
           bool TR = false>
-struct GemmDma {
-  static constexpr int TM = BM / WM / 32, TN = BN / WN / 32, TK = BK / 16;
-  static constexpr int KC = BK / 8;                       // A chunks per row
-  static constexpr int NCB = BN / 8;                      // B chunks per row
+struct GemmDma : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
+  typedef GemmTile<T, BM, BN, BK, WM, WN, NT, TR> G;
+  using G::TK, G::KC, G::NCB, G::A_ELEMS, G::STAGE, G::ASH, G::AMASK, G::RSH, G::RMASK;
   static constexpr int A_DMA = BM * KC / NT;              // copies per thread per stage
   static constexpr int B_DMA = BK * NCB / NT;
   static constexpr int D = A_DMA + B_DMA;
-  static constexpr int A_ELEMS = BM * BK, STAGE = BM * BK + BK * BN;
   static constexpr int LDS_BYTES = S * STAGE * 2;
-  static constexpr int ASH = KC >= 16 ? 0 : (KC == 8 ? 1 : (KC == 4 ? 2 : 3));
-  static constexpr int AMASK = (KC < 16 ? KC : 16) - 1;
-  static constexpr int RP = BN >= 128 ? 1 : 128 / BN;     // B rows per 256 bytes
-  static constexpr int RSH = RP == 1 ? 0 : (RP == 2 ? 1 : 2);
-  static constexpr int RMASK = 4 / RP - 1;
-  static_assert(TM >= 1 && TN >= 1 && TK >= 1, "tile too small for 32x32x16 MFMA");
   static_assert((BM * KC) % NT == 0 && (BK * NCB) % NT == 0, "tile/thread mismatch");
-  static_assert(WM * WN * 64 == NT, "warps must tile the block");
   static_assert(S >= 2 && (S - 2) * D <= 63, "vmcnt range");
-  static_assert(NCB >= 4 * (RMASK + 1), "B swizzle needs the row's chunks");
   static_assert(SPLIT >= 0 && SPLIT <= TK, "copies issue after SPLIT of the TK k slices");
-
-  static EK_INLINE int a_chunk(int row, int kc) { return row * KC + (kc ^ ((row >> ASH) & AMASK)); }
-  static EK_INLINE int b_chunk(int k, int nc) { return k * NCB + (nc ^ (((k >> RSH) & RMASK) << 2)); }
 
   // Per-thread copy plan, fixed for the whole loop: the global element offset of each chunk
   // relative to the k origin, or -1 when the chunk's column lies outside the operand.
@@ -949,47 +992,6 @@ struct GemmDma {
     }
   }
 
-  // One k slice: every A and B fragment read, then the TM x TN MFMAs.
-  EK_INLINE void compute_kk(int kk, float* acc, const uint16_t* st, int lane, int wm, int wn) {
-    typedef short v4s __attribute__((ext_vector_type(4)));
-    const u32x4* sA = reinterpret_cast<const u32x4*>(st);
-    const uint16_t* sB = st + A_ELEMS;
-    const int r32 = lane & 31, h = lane >> 5;
-    const int g = lane >> 4, ti = (lane >> 2) & 3, tq = lane & 3;
-    T a[TM][8], b[TN][8];
-    const int kc = kk * 2 + h;
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
-      const u32x4 v = sA[a_chunk(wm * (BM / WM) + tm * 32 + r32, kc)];
-      __builtin_memcpy(a[tm], &v, 16);
-    }
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const int n = wn * (BN / WN) + tn * 32 + 16 * (g & 1) + 4 * tq;
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const int k = kk * 16 + 8 * (g >> 1) + 4 * half + ti;
-        const uint16_t* src = sB + b_chunk(k, n >> 3) * 8 + (n & 7);
-        const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) v4s*)(src));
-        __builtin_memcpy(&b[tn][4 * half], &v, 8);
-      }
-    }
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) {
-        if constexpr (TR) mfma_32x32x16(&acc[(tm * TN + tn) * 16], b[tn], a[tm]);
-        else mfma_32x32x16(&acc[(tm * TN + tn) * 16], a[tm], b[tn]);
-      }
-  }
-
-  template <int KK0, int KK1>
-  EK_INLINE void compute(float* acc, const uint16_t* st, int lane, int wm, int wn) {
-#pragma unroll
-    for (int kk = KK0; kk < KK1; ++kk) compute_kk(kk, acc, st, lane, wm, wn);
-  }
-
   // Runs the whole k loop: k = lo, lo + BK, ... < hi.
   EK_INLINE void run(float* acc, const T* A, int lda, const T* B, int ldb, int M, int N, int K,
                      int m0, int n0, int lo, int hi, char* smem, int tid) {
@@ -1019,7 +1021,7 @@ struct GemmDma {
       // slice's reads, so each share's issue overlaps the MFMAs already queued (as one block
       // the copies kept the wave from issuing for 500-800 cycles per k step).
       const uint16_t* cur = s16 + (it % S) * STAGE;
-      compute<0, SPLIT>(acc, cur, lane, wm, wn);
+      G::template compute<0, SPLIT>(acc, cur, lane, wm, wn);
       if constexpr (SPLIT < TK) {
         constexpr int SL = TK - SPLIT, PER = (D + SL - 1) / SL;
         const int kn = lo + (it + S - 1) * BK;
@@ -1029,7 +1031,7 @@ struct GemmDma {
 #pragma unroll
           for (int j = q * PER; j < (q + 1) * PER && j < D; ++j)
             copy_one(j, ra, rb, ldb, K, kn, stn, wave);
-          compute_kk(SPLIT + q, acc, cur, lane, wm, wn);
+          G::compute_kk(SPLIT + q, acc, cur, lane, wm, wn);
         }
       } else {
         copy(ra, rb, ldb, K, lo + (it + S - 1) * BK, l0 + ((it + S - 1) % S) * STAGE * 2, wave);
