@@ -25,7 +25,8 @@ import sys
 import threading
 from pathlib import Path
 
-from enceladus_amd.compiler import codegen_hip, frontend, ir, rewrite, simplify, verify, widen
+from enceladus_amd.compiler import (codegen_hip, frontend, ir, pointer_gemm, rewrite,
+                                    simplify, verify, widen)
 from enceladus_amd.runtime import hip
 
 log = logging.getLogger("enceladus")
@@ -303,6 +304,9 @@ def build_module(jfn, arg_types, arg_facts, constexprs, num_warps, options) -> i
     if not (options or {}).get("no_simplify"):
         simplify.simplify(fn)
         verify.maybe_verify(fn, "the simplifier")
+    if not (options or {}).get("no_pointer_gemm") and pointer_gemm.lift_pointer_gemm(fn):
+        verify.maybe_verify(fn, "the pointer matmul rewrite")
+        ir.dce(fn)
     if widen.needs_idx64(fn):
         widen.widen_index_math(fn)
         verify.maybe_verify(fn, "64-bit index widening")

@@ -1,0 +1,89 @@
+"""Which pointer-and-mask loops become descriptor loops (CPU: the IR the pass leaves)."""
+
+import numpy as np
+import pytest
+
+import enceladus
+import enceladus.language as tl
+from enceladus_amd.compiler import ir
+
+H = np.zeros(16, np.float16)
+
+
+@enceladus.jit
+def _loop(a_ptr, b_ptr, c_ptr, M, N, K, sa, sb, sk, KIND: tl.constexpr, BM: tl.constexpr,
+          BN: tl.constexpr, BK: tl.constexpr):
+    pm, pn = tl.program_id(1), tl.program_id(0)
+    rm = pm * BM + tl.arange(0, BM)
+    if KIND == "swizzled":
+        rm = (pm // 2) * BM - BM + tl.arange(0, BM)
+    rn = pn * BN + tl.arange(0, BN)
+    rk = tl.arange(0, BK)
+    ap = a_ptr + rm[:, None] * sa + rk[None, :] * sk
+    bp = b_ptr + rk[:, None] * sb + rn[None, :]
+    acc = tl.zeros((BM, BN), dtype=tl.float32)
+    if KIND == "trips":
+        for k in range(0, tl.cdiv(K, BK)):
+            a = tl.load(ap, mask=(rm[:, None] < M) & (rk[None, :] < K - k * BK), other=0.0)
+            b = tl.load(bp, mask=(rk[:, None] < K - k * BK) & (rn[None, :] < N), other=0.0)
+            acc = tl.dot(a, b, acc)
+            ap += BK * sk
+            bp += BK * sb
+    elif KIND == "computed":
+        for k in range(0, K, BK):
+            a = tl.load(a_ptr + rm[:, None] * sa + (k + rk)[None, :] * sk,
+                        mask=(rm[:, None] < M) & ((k + rk)[None, :] < K), other=0.0)
+            b = tl.load(b_ptr + (k + rk)[:, None] * sb + rn[None, :],
+                        mask=((k + rk)[:, None] < K) & (rn[None, :] < N), other=0.0)
+            acc = tl.dot(a, b, acc)
+    elif KIND == "unmasked":
+        for k in range(0, K, BK):
+            acc = tl.dot(tl.load(ap), tl.load(bp), acc)
+            ap += BK * sk
+            bp += BK * sb
+    else:
+        for k in range(0, K, BK):
+            ma = (rm[:, None] < M) & (rk[None, :] + k < K)
+            mb = (rk[:, None] + k < K) & (rn[None, :] < N)
+            if KIND == "a_only":
+                b = tl.load(bp, mask=rn[None, :] < N, other=0.0)
+            elif KIND == "other":
+                b = tl.load(bp, mask=mb, other=1.0)
+            else:
+                b = tl.load(bp, mask=mb, other=0.0)
+            if KIND == "lower":
+                a = tl.load(ap, mask=ma & (rm[:, None] >= 3), other=0.0)
+            elif KIND == "shrinking":
+                a = tl.load(ap, mask=(rm[:, None] + k < M) & (rk[None, :] + k < K), other=0.0)
+            else:
+                a = tl.load(ap, mask=ma, other=0.0)
+            acc = tl.dot(a, b, acc)
+            if KIND == "half_step":
+                ap += (BK // 2) * sk
+            else:
+                ap += BK * sk
+            bp += BK * sb
+    cp = c_ptr + rm[:, None] * N + rn[None, :]
+    tl.store(cp, acc.to(tl.float16), mask=(rm[:, None] < M) & (rn[None, :] < N))
+
+
+LIFTED = ["plain", "trips", "computed", "unmasked", "swizzled"]
+KEPT = ["a_only", "other", "lower", "shrinking", "half_step"]
+
+
+def _ops(kind, dtype=H, sk=1, bm=64, bk=32):
+    f = _loop.ir(dtype, dtype, dtype, 100, 90, 70, 71, 91, sk, KIND=kind, BM=bm, BN=64, BK=bk)
+    return [op.name for op in ir.walk(f.body)]
+
+
+@pytest.mark.parametrize("kind", LIFTED + KEPT)
+def test_which_loops_are_lifted(kind):
+    names = _ops(kind)
+    assert (names.count("desc_load") == 2) == (kind in LIFTED)
+    assert (names.count("load") == 0) == (kind in LIFTED)
+
+
+def test_strided_k_wider_types_and_small_tiles_stay():
+    assert "desc_load" not in _ops("plain", sk=2)
+    assert "desc_load" not in _ops("plain", dtype=np.zeros(16, np.float32))
+    assert "desc_load" not in _ops("plain", bm=16)
