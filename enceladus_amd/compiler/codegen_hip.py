@@ -3237,7 +3237,7 @@ class Emitter:
     # -- dot loops on the GEMM template ---------------------------------------------------
     def _gemm_match(self, op):
         """Matches `for k in range(lo, hi, BK): acc = dot(dA.load([m0, k]), dB.load([k, n0]),
-        acc)` with loop-invariant m0/n0, 16-bit operands and aligned row-major tiles.
+        acc)` with loop-invariant m0/n0 and 16-bit or fp32 operands.
         Returns a dict for the template, or None to use the generic lowering."""
         body = op.regions[0]
         iv, carried = body.args[0], body.args[1:]
@@ -3283,7 +3283,7 @@ class Emitter:
         if la.operands[1].id in dep or lb.operands[2].id in dep:
             return None
         dt = a.type.dtype
-        if dt not in (core.float16, core.bfloat16) or b.type.dtype is not dt:
+        if dt not in (core.float16, core.bfloat16, core.float32) or b.type.dtype is not dt:
             return None
         if c.type.dtype is not core.float32:
             return None
@@ -3292,13 +3292,11 @@ class Emitter:
         bn = b.type.shape[1]
         if not (step.op is not None and step.op.name == "const" and step.op.attrs["value"] == bk):
             return None
-        plan = self.dot_plans[dot.result.id]
-        if plan.inst.m != 32 or plan.inst.k != 16 or plan.wrep != 1 or \
-                tuple(plan.korder) != tuple(range(len(plan.korder))):
+        plan = self.dot_plans.get(dot.result.id)
+        if plan is None or plan.inst.m != 32 or plan.inst.k != (2 if dt is core.float32 else 16) or \
+                plan.wrep != 1 or tuple(plan.korder) != tuple(range(len(plan.korder))):
             return None
-        nt = self.nt
-        kc = bk // 8
-        if bk % 16:
+        if bk % 16 or 2 * (bm + bn) * bk * dt.itemsize > MAX_LDS:
             return None
         if self.lay[acc.id].key() != LY.mfma_acc(plan).key():
             return None
@@ -3334,8 +3332,8 @@ class Emitter:
         whole = rows and all(div(v) % 8 == 0 for v in (A["shape_v"][1], B["shape_v"][1]))
         buf = not (big or not whole or self.opt.get("no_buffer_loads"))
         bm, bn, bk = g["bm"], g["bn"], g["bk"]
-        stage = (bm * bk + bk * bn) * 2
-        dma = (buf and not self.opt.get("no_lds_dma") and (bm * bk // 8) % self.nt == 0
+        stage = (bm * bk + bk * bn) * g["dt"].itemsize
+        dma = (buf and g["dt"] is not core.float32 and not self.opt.get("no_lds_dma") and (bm * bk // 8) % self.nt == 0
                and (bk * bn // 8) % self.nt == 0 and bn >= 32)
         if dma:
             # Stages: as many (at most 4) as fit the LDS share of a workgroup when a CU keeps
@@ -3351,6 +3349,7 @@ class Emitter:
                     f"{split}{tr}>")
             self.need_lds(nst * stage)
         else:
+            rows = rows and g["dt"] is not core.float32
             tmpl = (f"ek::{'Gemm' if rows else 'GemmReg'}<{T}, {bm}, {bn}, {bk}, {p.wm}, {p.wn}, "
                     f"{self.nt}, {'true' if big else 'false'}{', true' if p.trans else ''}>")
             self.need_lds(2 * stage)

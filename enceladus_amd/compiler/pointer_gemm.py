@@ -39,7 +39,7 @@ from __future__ import annotations
 from enceladus_amd.compiler import ir
 from enceladus_amd.language import core
 
-_HALF = (core.float16, core.bfloat16)
+_DTYPES = (core.float16, core.bfloat16, core.float32)
 _BODY_OPS = ir.PURE_OPS | {"load", "dot", "yield"}
 _MAX_TERMS = 16
 
@@ -255,7 +255,7 @@ class _Loop:
         if any(len(self.uses.get(x.result.id, [])) != 1 for x in loads):
             return False
         dt = la.result.type.dtype
-        if dt not in _HALF or lb.result.type.dtype is not dt or \
+        if dt not in _DTYPES or lb.result.type.dtype is not dt or \
                 dot.result.type.dtype is not core.float32:
             return False
         (bm, bk), bn = la.result.type.shape, lb.result.type.shape[1]

@@ -684,6 +684,8 @@ EK_INLINE void dma16(i32x4 rsrc, uint32_t lds, int voff) {
 // ---------------------------------------------------------------------------
 template <typename T, int BM, int BN, int BK, int WM, int WN, int NT, bool TR>
 struct GemmTile {
+  typedef uint16_t E;                                     // an element in LDS
+  static constexpr int EC = 8;                            // elements per chunk
   static constexpr int TM = BM / WM / 32, TN = BN / WN / 32, TK = BK / 16;
   static constexpr int KC = BK / 8;                       // A chunks per row
   static constexpr int NCB = BN / 8;                      // B chunks per row
@@ -742,6 +744,58 @@ struct GemmTile {
   }
 };
 
+// The same for fp32 operands: 16-byte chunks of 4 elements, v_mfma_f32_32x32x2_f32 (one element
+// per lane: lanes 32..63 hold the odd k of a pair). A fragments are 16-byte reads, four k of a
+// row at a time (both halves of the wave read the same chunk and pick their k); B's are one
+// word per lane from two neighbouring rows, whose 128-byte runs the swizzle keeps in different
+// halves of the banks. The pairs run in k order, as the dot's own lowering has them.
+template <int BM, int BN, int BK, int WM, int WN, int NT, bool TR>
+struct GemmTile<float, BM, BN, BK, WM, WN, NT, TR> {
+  typedef float E;
+  static constexpr int EC = 4;
+  static constexpr int TM = BM / WM / 32, TN = BN / WN / 32, TK = BK / 4;
+  static constexpr int KC = BK / 4, NCB = BN / 4;
+  static constexpr int A_ELEMS = BM * BK, STAGE = BM * BK + BK * BN;
+  static constexpr int ASH = KC >= 16 ? 0 : (KC == 8 ? 1 : 2);
+  static constexpr int AMASK = (KC < 16 ? KC : 16) - 1;
+  static constexpr int ODD = NCB >= 16 ? 8 : 0;
+  static_assert(!TR, "fp32 dots keep the instruction's orientation");
+  static_assert(TM >= 1 && TN >= 1 && KC >= 4, "tile too small for 32x32x2 MFMA");
+  static_assert(WM * WN * 64 == NT, "warps must tile the block");
+
+  static EK_INLINE int a_chunk(int row, int kc) { return row * KC + (kc ^ ((row >> ASH) & AMASK)); }
+  static EK_INLINE int b_chunk(int k, int nc) { return k * NCB + (nc ^ ((k & 1) * ODD)); }
+
+  template <int KK0, int KK1>
+  EK_INLINE void compute(float* acc, const float* st, int lane, int wm, int wn) {
+    const f32x4* sA = reinterpret_cast<const f32x4*>(st);
+    const float* sB = st + A_ELEMS;
+    const int r32 = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int q = KK0; q < KK1; ++q) {
+      f32x4 a[TM];
+      float b[2][TN];
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) a[tm] = sA[a_chunk(wm * (BM / WM) + tm * 32 + r32, q)];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) {
+          const int n = wn * (BN / WN) + tn * 32 + r32;
+          b[j][tn] = sB[b_chunk(q * 4 + 2 * j + h, n >> 2) * 4 + (n & 3)];
+        }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+          const float av = h ? a[tm][2 * j + 1] : a[tm][2 * j];
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn) mfma_32x32x2(&acc[(tm * TN + tn) * 16], &av, &b[j][tn]);
+        }
+    }
+  }
+};
+
 // ---------------------------------------------------------------------------
 // The loop for operands of any alignment and size, through registers: each thread loads its
 // 16-byte chunks of the tile PD steps ahead (element-aligned vector loads) and writes the tile
@@ -758,25 +812,27 @@ struct GemmTile {
 template <typename T, int BM, int BN, int BK, int WM, int WN, int NT, bool BIG, bool TR = false>
 struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
   typedef GemmTile<T, BM, BN, BK, WM, WN, NT, TR> G;
-  using G::TK, G::KC, G::NCB, G::A_ELEMS, G::STAGE;
+  using G::TK, G::KC, G::NCB, G::A_ELEMS, G::STAGE, G::EC;
+  typedef typename G::E E;
+  static constexpr int ES = sizeof(E);
   static constexpr int A_TOT = BM * KC, B_TOT = BK * NCB;
   static constexpr int A_CH = (A_TOT + NT - 1) / NT, B_CH = (B_TOT + NT - 1) / NT;
   static constexpr int CH = A_CH + B_CH;
   // k steps of loads in flight: about 32 registers' worth (64x64x32 tiles on 4 waves, bf16
   // 1000 x 3000 x 2000: 35.6 us at 4 steps, 38.9 at 1; 256x256x64 on 8 waves spills at 2)
   static constexpr int PD = CH <= 2 ? 4 : CH <= 4 ? 2 : 1;
-  static constexpr int LDS_BYTES = 2 * STAGE * 2;
+  static constexpr int LDS_BYTES = 2 * STAGE * ES;
   // byte offsets from a tile's k origin: 32 bits, or 64 for operands of 2 GiB and more
   template <bool> struct off_of { typedef uint32_t type; };
   template <> struct off_of<true> { typedef int64_t type; };
   typedef typename off_of<BIG>::type Off;
-  typedef u32x4 chunk __attribute__((aligned(2)));
+  typedef typename raw_u<E, EC>::type chunk;
 
   u32x4 r[PD][CH];
-  // Of each chunk, from a k step's first column less 8 (A: a chunk moved back from a ragged
-  // end starts up to 7 columns before it) or first row (B).
+  // Of each chunk, from a k step's first column less EC (A: a chunk moved back from a ragged
+  // end starts up to EC - 1 columns before it) or first row (B).
   Off off[CH], last[CH];    // of every k step, and of the last one
-  int sh[CH], lsh[CH];      // elements to shift (8 and more: all zero), likewise
+  int sh[CH], lsh[CH];      // elements to shift (EC and more: all zero), likewise
 
   static EK_INLINE int row_a(int i, int tid) { return (i * NT + tid) / KC; }
   static EK_INLINE int kc_a(int i, int tid) { return (i * NT + tid) % KC; }
@@ -791,21 +847,21 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
   EK_INLINE void plan(int lda, int ldb, int M, int N, int K, int m0, int n0, int klast, int tid) {
 #pragma unroll
     for (int i = 0; i < A_CH; ++i) {
-      const int row = m0 + row_a(i, tid), rc = Min::op<int>(row, M - 1), c = kc_a(i, tid) * 8;
-      const int cl = Min::op<int>(klast + c, K - 8) - klast;     // -7 and more
-      off[i] = ((Off)rc * (Off)lda + (Off)(c + 8)) * 2;
-      last[i] = ((Off)rc * (Off)lda + (Off)(cl + 8)) * 2;
-      sh[i] = row < M ? 0 : 8;
-      lsh[i] = row < M ? c - cl : 8;
+      const int row = m0 + row_a(i, tid), rc = Min::op<int>(row, M - 1), c = kc_a(i, tid) * EC;
+      const int cl = Min::op<int>(klast + c, K - EC) - klast;    // 1 - EC and more
+      off[i] = ((Off)rc * (Off)lda + (Off)(c + EC)) * ES;
+      last[i] = ((Off)rc * (Off)lda + (Off)(cl + EC)) * ES;
+      sh[i] = row < M ? 0 : EC;
+      lsh[i] = row < M ? c - cl : EC;
     }
 #pragma unroll
     for (int j = 0; j < B_CH; ++j) {
-      const int i = A_CH + j, k = row_b(j, tid), gn = n0 + nc_b(j, tid) * 8;
-      const int kl = Min::op<int>(klast + k, K - 1) - klast, nl = Min::op<int>(gn, N - 8);
-      off[i] = ((Off)k * (Off)ldb + (Off)nl) * 2;
-      last[i] = ((Off)kl * (Off)ldb + (Off)nl) * 2;
+      const int i = A_CH + j, k = row_b(j, tid), gn = n0 + nc_b(j, tid) * EC;
+      const int kl = Min::op<int>(klast + k, K - 1) - klast, nl = Min::op<int>(gn, N - EC);
+      off[i] = ((Off)k * (Off)ldb + (Off)nl) * ES;
+      last[i] = ((Off)kl * (Off)ldb + (Off)nl) * ES;
       sh[i] = gn - nl;
-      lsh[i] = kl == k ? gn - nl : 8;
+      lsh[i] = kl == k ? gn - nl : EC;
     }
   }
 
@@ -817,7 +873,7 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
     }
   }
 
-  EK_INLINE void put(int p, uint16_t* st, int tid) {
+  EK_INLINE void put(int p, E* st, int tid) {
     u32x4* sA = reinterpret_cast<u32x4*>(st);
     u32x4* sB = reinterpret_cast<u32x4*>(st + A_ELEMS);
 #pragma unroll
@@ -833,15 +889,15 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
     for (int i = 0; i < CH; ++i) {
       const int s = end ? lsh[i] : sh[i];
       unsigned __int128 x = __builtin_bit_cast(unsigned __int128, r[p][i]);
-      x = s >= 8 ? 0 : x >> (16 * (s & 7));
+      x = s >= EC ? 0 : x >> (8 * ES * (s & (EC - 1)));
       r[p][i] = __builtin_bit_cast(u32x4, x);
     }
   }
 
   // One element of an operand [rows, cols], zero outside it.
-  static EK_INLINE uint16_t at(const T* P, int64_t ld, int rows, int cols, int i, int j) {
+  static EK_INLINE E at(const T* P, int64_t ld, int rows, int cols, int i, int j) {
     if (i < 0 || i >= rows || j < 0 || j >= cols) return 0;
-    return reinterpret_cast<const uint16_t*>(P)[i * ld + j];
+    return reinterpret_cast<const E*>(P)[i * ld + j];
   }
 
   // Runs the whole k loop: k = lo, lo + BK, ... < hi.
@@ -852,19 +908,19 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
     const int niter = (int)(((int64_t)hi - lo + BK - 1) / BK);
     const int lane = tid & 63, warp = tid >> 6;
     const int wm = warp % WM, wn = warp / WM;
-    uint16_t* s16 = reinterpret_cast<uint16_t*>(smem);
+    E* sm = reinterpret_cast<E*>(smem);
     __syncthreads();  // earlier users of the LDS are done with it
-    if (m0 < 0 || n0 < 0 || lo < 0 || M < 1 || N < 8 || K < 8) {
+    if (m0 < 0 || n0 < 0 || lo < 0 || M < 1 || N < EC || K < EC) {
       for (int it = 0; it < niter; ++it) {
         const int k = lo + it * BK;
         for (int c = tid; c < BM * BK; c += NT)
-          s16[G::a_chunk(c / BK, (c % BK) / 8) * 8 + c % 8] =
+          sm[G::a_chunk(c / BK, (c % BK) / EC) * EC + c % EC] =
               at(A, lda, M, K, m0 + c / BK, k + c % BK);
         for (int c = tid; c < BK * BN; c += NT)
-          s16[A_ELEMS + G::b_chunk(c / BN, (c % BN) / 8) * 8 + c % 8] =
+          sm[A_ELEMS + G::b_chunk(c / BN, (c % BN) / EC) * EC + c % EC] =
               at(B, ldb, K, N, k + c / BN, n0 + c % BN);
         __syncthreads();
-        G::template compute<0, TK>(acc, s16, lane, wm, wn);
+        G::template compute<0, TK>(acc, sm, lane, wm, wn);
         __syncthreads();
       }
       return;
@@ -872,9 +928,9 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
     const int klast = lo + (niter - 1) * BK;
     const bool edge = m0 + BM > M || n0 + BN > N, ragged = klast + BK > K;
     plan(lda, ldb, M, N, K, m0, n0, klast, tid);
-    const char* a = reinterpret_cast<const char*>(A) + ((int64_t)lo - 8) * 2;
-    const char* b = reinterpret_cast<const char*>(B) + (int64_t)lo * ldb * 2;
-    const int64_t sa = BK * 2, sb = (int64_t)BK * ldb * 2;
+    const char* a = reinterpret_cast<const char*>(A) + ((int64_t)lo - EC) * ES;
+    const char* b = reinterpret_cast<const char*>(B) + (int64_t)lo * ldb * ES;
+    const int64_t sa = BK * ES, sb = (int64_t)BK * ldb * ES;
 #pragma unroll
     for (int p = 0; p < PD; ++p) {
       const int t = Min::op<int>(p, niter - 1);
@@ -887,7 +943,7 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
         if (t >= niter) break;
         const bool end = t == niter - 1;
         if (edge || (end && ragged)) shift(p, end);
-        uint16_t* st = s16 + (PD % 2 ? (t & 1) : (p & 1)) * STAGE;
+        E* st = sm + (PD % 2 ? (t & 1) : (p & 1)) * STAGE;
         put(p, st, tid);
         // past the end: the last tile again, which nothing reads
         const int nx = Min::op<int>(t + PD, niter - 1);

@@ -29,3 +29,15 @@ def test_any_size_and_alignment(mnk, tile, lead):
     bm, bn, bk, nw = tile
     c = matmul_desc(a, b, bm=bm, bn=bn, bk=bk, num_warps=nw)
     assert np.array_equal(c.double().cpu().numpy(), want.numpy())
+
+
+@pytest.mark.parametrize("tile", [(32, 32, 16, 1), (64, 64, 32, 4), (128, 128, 64, 4),
+                                  (256, 128, 32, 8), (128, 32, 16, 4)])
+@pytest.mark.parametrize("mnk", [(1, 1, 1), (5, 3, 7), (64, 4, 4), (65, 71, 130), (257, 132, 500)])
+@pytest.mark.parametrize("lead", [0, 1])
+def test_any_size_and_alignment_fp32(mnk, tile, lead):
+    m, n, k = mnk
+    a, b = whole(m, k, 1, lead, "float32"), whole(k, n, 2, lead, "float32")
+    bm, bn, bk, nw = tile
+    c = matmul_desc(a, b, bm=bm, bn=bn, bk=bk, num_warps=nw)
+    assert np.array_equal(c.double().cpu().numpy(), (a.double() @ b.double()).cpu().numpy())
