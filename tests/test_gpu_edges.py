@@ -88,3 +88,25 @@ def test_layout_conversions_larger_than_the_lds(shape, dtype):
     o = torch.zeros(n, m, dtype=x.dtype, device="cuda")
     _transpose[(1,)](x, o, M=m, N=n, num_warps=8)
     assert torch.equal(o, x.t())
+
+
+@enceladus.jit
+def _cyclic(t_ptr, o_ptr, start, n, BLOCK: tl.constexpr):
+    i = tl.program_id(0) * BLOCK + tl.arange(0, BLOCK)
+    tl.store(o_ptr + i, tl.load(t_ptr + (start + i) % n))
+
+
+@pytest.mark.parametrize("dtype", ["int8", "float16", "float32"])
+@pytest.mark.parametrize("n", [1, 2, 3, 7, 8, 33, 1000, 1023, 1024, 1025, 4099, 100000])
+@pytest.mark.parametrize("start", [0, 1, 5000, -1500])
+def test_cyclic_loads(n, start, dtype):
+    """`table + x % n` (C's remainder) for tiles inside one period, across its end, over many
+    periods, and of negative x."""
+    import torch
+    size, pad = 3 * 1024, n
+    table = torch.arange(2 * n + 1).remainder(113).to(getattr(torch, dtype)).cuda()
+    out = torch.zeros(size, dtype=table.dtype, device="cuda")
+    _cyclic[(3,)](table[pad:], out, start, n, BLOCK=1024)
+    x = np.arange(start, start + size)
+    want = table.cpu()[torch.from_numpy(pad + np.fmod(x, n))]
+    assert torch.equal(out.cpu(), want)
