@@ -302,11 +302,12 @@ class Emitter:
         self.emit(f"}} else if ({q}r >= 0 && {nn} >= {V}) {{")
         self._vec_loop(lay.nregs, V)
         self.emit(f"  const int ek_r = (int)((uint32_t)({q}x + {c}) % (uint32_t){nn});")
-        self.emit(f"  if (ek_r <= {nn} - {V}) ek::vload_u<{t}, {V}>(&{nm}[rv], {b} + ek_r);")
-        self.emit("  else {")
-        for i in range(V):
-            self.emit(f"    {nm}[rv + {i}] = {b}[ek_r + {i} < {nn} ? ek_r + {i} : ek_r + {i} - "
-                      f"{nn}];")
+        self.emit(f"  const int ek_s = ek_r - ek::Min::op<int>(ek_r, {nn} - {V});")
+        self.emit(f"  ek::vload_u<{t}, {V}>(&{nm}[rv], {b} + (ek_r - ek_s));")
+        self.emit("  if (__builtin_amdgcn_ballot_w64(ek_s > 0) != 0) {")
+        self.emit(f"    {t} ek_w[{V}];")
+        self.emit(f"    ek::vload_u<{t}, {V}>(ek_w, {b});")
+        self.emit(f"    ek::wrap_shift<{t}, {V}>(&{nm}[rv], ek_s, ek_w);")
         self.emit("  }")
         self.emit("}")
         self.emit("} else {")

@@ -276,6 +276,18 @@ template <typename T, int V> EK_INLINE void edge_shift(T* v, int s, const T* o) 
   for (int i = 0; i < V; ++i) v[i] = s >= V ? o[i] : v[i];
 }
 
+// The V elements that start s < V elements into `v` and go on, past its end, with the first
+// ones of `w`.
+template <typename T, int V> EK_INLINE void wrap_shift(T* v, int s, const T* w) {
+  typedef typename bits_of<sizeof(T) * V>::type U;
+  constexpr int B = sizeof(T) * 8;
+  U x, y;
+  __builtin_memcpy(&x, v, sizeof(U));
+  __builtin_memcpy(&y, w, sizeof(U));
+  if (s > 0) x = (U)(x >> (B * s)) | (U)(y << (B * (V - s)));
+  __builtin_memcpy(v, &x, sizeof(U));
+}
+
 // ---------------------------------------------------------------------------
 // Wave64 cross-lane moves.
 // ---------------------------------------------------------------------------
