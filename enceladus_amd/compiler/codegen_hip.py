@@ -150,6 +150,10 @@ class GeneratedKernel:
     # indices), "total" (words per workgroup row of the partial buffer), "chunks" (64-word
     # column chunks)}; the launcher runs `name` on grid (chunks, rows / rb) after the kernel
     flush: dict | None = None
+    # a block GEMM that may be split along k: {"hi" (index of the argument that bounds k), "bk",
+    # "words" (floats of one workgroup's accumulator), "step_us" (a k step's time, roughly)}; its last argument is the workspace
+    # (0: not split), and a split launch runs one workgroup per tile and slice (grid z)
+    split: dict | None = None
     # what `kernel.explain` reports: {"conversions", "lds", "dots"} recorded by the emitter
     report: dict = field(default_factory=dict)
 
@@ -187,6 +191,7 @@ class Emitter:
         self.fast_streams = 0
         self.fast_failed = False
         self.edge_only = False       # the general copy runs only for edge programs
+        self.split: dict | None = None
 
     # ------------------------------------------------------------------ utilities
     def fresh(self, hint="v") -> str:
@@ -3368,6 +3373,25 @@ class Emitter:
         return {"plan": plan, "A": A, "B": B, "m0": la.operands[1], "n0": lb.operands[2],
                 "scalar_ops": scalar_ops, "dt": dt, "bm": bm, "bn": bn, "bk": bk}
 
+    def _can_split(self, op) -> bool:
+        """Whether the block GEMM loop `op` may run in slices of k on several workgroups: it is
+        the program's only loop, at the top level, from 0 to an argument; nothing before it has
+        a side effect (every slice runs it); and the program has no third grid axis, which
+        the slices take."""
+        body = self.fn.body.ops
+        if self.opt.get("no_split_k") or op not in body or self.coarsen or self.priv or \
+                op.operands[1] not in self.fn.args or \
+                op.operands[1].type.dtype is not core.int32 or \
+                self._const_of(op.operands[0]) != 0:
+            return False
+        names = [o.name for o in ir.walk(self.fn.body)]
+        if names.count("for") != 1 or "assert" in names or "print" in names or any(
+                o.name in ("program_id", "num_programs") and o.attrs.get("axis", 0) == 2
+                for o in ir.walk(self.fn.body)):
+            return False
+        return all(o.name in ir.PURE_OPS or o.name in ("load", "make_desc", "desc_load")
+                   for o in body[:body.index(op)])
+
     def _emit_gemm_loop(self, op, g) -> bool:
         self.report["gemm_template"] = op.loc
         body = op.regions[0]
@@ -3417,10 +3441,33 @@ class Emitter:
             tmpl = (f"ek::{'Gemm' if rows else 'GemmReg'}<{T}, {bm}, {bn}, {bk}, {p.wm}, {p.wn}, "
                     f"{self.nt}, {'true' if big else 'false'}{', true' if p.trans else ''}>")
             self.need_lds(2 * stage)
+        if self._can_split(op):
+            # a k step's time on a CU of an otherwise idle chip: its bytes at about 20 us a
+            # MB (64x64x128 fp16: 0.65 us measured), or its MFMAs at half their peak
+            # (128x128x64 fp32: 5.2 us)
+            rate = 0.4e6 if g["dt"] is core.float32 else 4.9e6
+            self.split = {"hi": next(i for i, a in enumerate(self.fn.args)
+                                     if a is op.operands[1]), "bk": bk,
+                          "words": lay.nregs * self.nt,
+                          "step_us": round(max(2e-5 * stage, 2 * bm * bn * bk / rate), 3)}
+            self.emit(f"  int ek_lo = {lo}, ek_hi = {hi};")
+            self.emit("  if (ek_ws) {")
+            self.emit(f"    const int ek_per = ek::split_slice(ek_lo, ek_hi, {bk}, gridDim.z);")
+            self.emit("    ek_lo += (int)blockIdx.z * ek_per;")
+            self.emit("    ek_hi = ek::Min::op<int>(ek_hi, ek_lo + ek_per);")
+            self.emit("    if (blockIdx.z) {")
+            self.emit("      #pragma unroll")
+            self.emit(f"      for (int r = 0; r < {lay.nregs}; ++r) {nm}[r] = 0.0f;")
+            self.emit("    }")
+            self.emit("  }")
+            lo, hi = "ek_lo", "ek_hi"
         self.emit(f"  {tmpl} ek_g;")
         self.emit(f"  ek_g.run({nm}, {A['base']}, {A['strides'][0]}, {B['base']}, "
                   f"{B['strides'][0]}, {A['shape'][0]}, {B['shape'][1]}, {A['shape'][1]}, "
                   f"{self.name[g['m0'].id]}, {self.name[g['n0'].id]}, {lo}, {hi}, ek_smem, ek_tid);")
+        if self.split:
+            self.emit(f"  if (ek_ws && !ek::split_reduce<{lay.nregs}, {self.nt}>({nm}, ek_ws, "
+                      "ek_smem, ek_tid)) return;")
         self.emit("}")
         self.define(op.results[0], nm)
         self.big_acc = max(getattr(self, "big_acc", 0), lay.nregs)
@@ -3753,6 +3800,9 @@ class Emitter:
         if self.asserts:
             params.append("uint32_t* ek_assert_buf")
             args.append(KernelArg("ek_assert_buf", "ptr", core.uint32, "uint32_t*"))
+        if self.split:
+            params.append("float* ek_ws")
+            args.append(KernelArg("ek_ws", "ptr", core.float32, "float*"))
         # Two-level flush of privatised bins: each workgroup stores its bins to a partial
         # buffer row (plain stores), and a second kernel sums a block of RB rows by 64 words
         # and adds each sum with one global atomic. Measured on the 1024-bin histogram: one
@@ -3926,6 +3976,7 @@ class Emitter:
         gk.coarsen = int(self.coarsen)
         gk.asserts = list(self.asserts)
         gk.flush = flush
+        gk.split = self.split
         gk.report = self.report
         return gk
 

@@ -8,7 +8,10 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 // The HIP runtime's launch with dispatch-boundary events (declared in hip/hip_ext.h, whose
@@ -36,6 +39,11 @@ int check(hipError_t e, const char* what, char* err, size_t errlen) {
                     hipGetErrorString(e) + ")";
   return fail(err, errlen, msg);
 }
+
+// Workspaces of split launches: one per (device, stream), of one fixed size (a launch in
+// progress on another thread never sees its workspace move), at most EK_WORKSPACES of them.
+std::mutex g_ws_lock;
+std::map<std::pair<int, hipStream_t>, void*> g_ws;
 
 #define EK_CHECK(call) \
   do { if (int _rc = check((call), #call, err, errlen)) return _rc; } while (0)
@@ -200,7 +208,66 @@ int ek_stream_new(void** stream, char* err, size_t errlen) {
   return 0;
 }
 
+int ek_workspace(void* stream, void** ptr, char* err, size_t errlen) {
+  *ptr = nullptr;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipStreamIsCapturing(s, &cap) != hipSuccess ||
+      cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  std::lock_guard<std::mutex> hold(g_ws_lock);
+  auto it = g_ws.find({dev, s});
+  if (it != g_ws.end()) {
+    *ptr = it->second;
+    return 0;
+  }
+  if (g_ws.size() >= EK_WORKSPACES) return 0;
+  void* p = nullptr;
+  if (hipMalloc(&p, EK_WORKSPACE_BYTES) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  // the counters start at zero, and every launch leaves them there
+  if (hipMemset(p, 0, EK_WORKSPACE_BYTES) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+    (void)hipFree(p);
+    return fail(err, errlen, "ek_workspace: clearing the workspace failed");
+  }
+  g_ws[{dev, s}] = p;
+  *ptr = p;
+  return 0;
+}
+
+int ek_workspace_release(char* err, size_t errlen) {
+  std::lock_guard<std::mutex> hold(g_ws_lock);
+  int here = 0;
+  EK_CHECK(hipGetDevice(&here));
+  for (auto& e : g_ws) {
+    EK_CHECK(hipSetDevice(e.first.first));
+    EK_CHECK(hipDeviceSynchronize());
+    EK_CHECK(hipFree(e.second));
+    e.second = nullptr;
+  }
+  g_ws.clear();
+  EK_CHECK(hipSetDevice(here));
+  return 0;
+}
+
 int ek_stream_free(void* stream, char* err, size_t errlen) {
+  {
+    std::lock_guard<std::mutex> hold(g_ws_lock);
+    for (auto it = g_ws.begin(); it != g_ws.end();) {
+      if (it->first.second != static_cast<hipStream_t>(stream) || !stream) {
+        ++it;
+        continue;
+      }
+      EK_CHECK(hipStreamSynchronize(it->first.second));
+      EK_CHECK(hipFree(it->second));
+      it = g_ws.erase(it);
+    }
+  }
   EK_CHECK(hipStreamDestroy(static_cast<hipStream_t>(stream)));
   return 0;
 }

@@ -1110,4 +1110,77 @@ struct GemmDma : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
   }
 };
 
+// ---------------------------------------------------------------------------
+// Split k loops. A grid with few tiles leaves most CUs idle while each workgroup walks the
+// whole k range, one tile's latency after another; the launcher then starts ns = gridDim.z
+// workgroups per tile, each on a slice of k. Every workgroup stores its accumulator (registers
+// as they are, NT lanes side by side) to its row of the workspace and counts itself in; the
+// last one of a tile adds all rows in slice order (so the sum does not depend on who is last),
+// clears the tile's counter for the next launch and returns true: it runs the epilogue.
+//
+// The partial rows go through relaxed agent-scope atomics, which write to and read from memory
+// past the XCDs' private L2s; a vmcnt wait before the count makes sure that they are there. That
+// costs the rows alone, where an agent-scope release or acquire fence writes back or drops
+// a whole L2.
+// ---------------------------------------------------------------------------
+constexpr int kSplitCounters = 16384;     // words at the start of the workspace: one per tile
+
+EK_INLINE int split_slice(int lo, int hi, int bk, int ns) {   // k extent of one slice
+  const int steps = (hi - lo + bk - 1) / bk;
+  return (steps + ns - 1) / ns * bk;
+}
+
+template <int R, int NT>
+EK_INLINE bool split_reduce(float* acc, float* ws, char* smem, int tid) {
+  constexpr int P = R / 2;                // pairs of accumulator registers: 8-byte accesses
+  constexpr int U = R <= 16 ? 4 : R <= 64 ? 2 : 1;   // rows in flight while they are added
+  static_assert(R % 2 == 0, "pairs of registers");
+  const int ns = gridDim.z, tile = blockIdx.x + gridDim.x * blockIdx.y;
+  uint32_t* count = reinterpret_cast<uint32_t*>(ws) + tile;
+  uint64_t* rows = reinterpret_cast<uint64_t*>(ws + kSplitCounters) +
+                   (int64_t)tile * ns * (P * NT) + tid;
+  uint64_t* mine = rows + (int64_t)blockIdx.z * (P * NT);
+#pragma unroll
+  for (int r = 0; r < P; ++r) {
+    uint64_t v;
+    __builtin_memcpy(&v, &acc[2 * r], 8);
+    __hip_atomic_store(mine + r * NT, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  uint32_t* last = reinterpret_cast<uint32_t*>(smem);
+  __syncthreads();   // every lane's rows are in memory; the LDS is free
+  if (tid == 0)
+    *last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+            (uint32_t)ns - 1;
+  __syncthreads();
+  if (*last == 0) return false;
+  if (tid == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+  for (int z = 0; z < ns; z += U) {
+    uint64_t part[U][P];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int zr = z + u < ns ? z + u : ns - 1;
+#pragma unroll
+      for (int r = 0; r < P; ++r)
+        part[u][r] = __hip_atomic_load(rows + (int64_t)zr * (P * NT) + r * NT, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (z + u >= ns) break;
+#pragma unroll
+      for (int r = 0; r < P; ++r) {
+        float v[2];
+        __builtin_memcpy(v, &part[u][r], 8);
+        acc[2 * r] += v[0];
+        acc[2 * r + 1] += v[1];
+      }
+    }
+  }
+  __syncthreads();   // `last` is read; the epilogue may use the LDS
+  return true;
+}
+
 }  // namespace ek

@@ -145,8 +145,8 @@ class CompiledKernel:
 
     def pack(self, values) -> bytes:
         values = list(values)
-        if self.gen.flush:
-            values.append(0)      # the partial-bin buffer, set per stream at launch
+        if self.gen.flush or self.gen.split:
+            values.append(0)      # the partial-bin buffer or workspace, set per stream at launch
         b = codegen_hip.pack_args(self.args, values, pad8=not self.gen.coarsen)
         self.packed_size = len(b)
         return b
@@ -186,6 +186,16 @@ class CompiledKernel:
             kernarg += b"\0" * ((-len(kernarg)) % 8)
         out = []
         fl = self.gen.flush
+        if self.gen.split and gz == 1:
+            import struct
+            offs = codegen_hip.arg_offsets(self.args)
+            hi = struct.unpack_from("<i", kernarg, offs[self.gen.split["hi"]])[0]
+            n = split_factor(self.gen.split, gx * gy, hi)
+            ws = workspace(stream) if n > 1 else 0
+            if ws:
+                kb = bytearray(kernarg)
+                struct.pack_into("<Q", kb, offs[-1], ws)
+                kernarg, gz = bytes(kb), n
         if fl:
             import struct
             offs = codegen_hip.arg_offsets(self.args)
@@ -273,6 +283,39 @@ def coarsen_cap() -> int:
         except Exception:  # noqa: BLE001
             _CAP = 256
     return _CAP
+
+
+def split_factor(split: dict, tiles: int, hi: int) -> int:
+    """Over how many workgroups per tile a block GEMM's k loop is split (1: it is not).
+
+    Only grids that leave at least half of the CUs without a workgroup and loops of 15 us
+    and more split, into slices of about 5 us and at most two workgroups per CU: shorter ones cost more in prologues and
+    partial rows than they save (fp16 64 x 4096 x 4096, 64 tiles: 21.6 us unsplit, 15.6 over 2,
+    13.6 over 4, 15.6 over 8, 21.7 over 16; K = 8192 on 16 tiles: 27.6, 17.9, 12.9, 12.4,
+    15.2; fp32 512 x 1024 x 1024, 32 tiles: 84.5, 49.7, 32.6 over 1, 2, 4). The rows have
+    to fit the workspace."""
+    cus = coarsen_cap()
+    steps = -(-hi // split["bk"])
+    n = int(steps * split["step_us"] / 5)
+    if n < 3 or tiles <= 0 or 2 * tiles > cus:
+        return 1
+    room = (hip.WORKSPACE_BYTES // 4 - hip.SPLIT_COUNTERS) // (tiles * split["words"])
+    return max(1, min(2 * cus // tiles, n, steps // 2, room))
+
+
+_ws_tls = threading.local()
+
+
+def workspace(stream: int) -> int:
+    """The device address of `stream`'s split workspace, or 0 when it has none (captured
+    streams, too many streams): the launch then does not split."""
+    t = _ws_tls
+    if not hasattr(t, "ptr"):
+        t.ptr, t.err = ctypes.c_void_p(), ctypes.create_string_buffer(1024)
+        t.ref, t.fn = ctypes.byref(t.ptr), hip.load_library().ek_workspace
+    if t.fn(stream or None, t.ref, t.err, 1024):
+        raise hip.HipError(f"ek_workspace: {t.err.value.decode(errors='replace')}")
+    return t.ptr.value or 0
 
 
 def compile_ir(fn: ir.Func, options: dict | None = None) -> CompiledKernel:

@@ -90,6 +90,8 @@ _SIGS = {
     "ek_launch_timed_events": [ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_uint32] * 7 +
                               [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p,
                                ctypes.c_void_p],
+    "ek_workspace": [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)],
+    "ek_workspace_release": [],
     "ek_launch_flush_noalloc": [ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_uint32] * 4 +
                                [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_size_t,
                                 ctypes.c_void_p] + [ctypes.c_uint32] * 3 +
@@ -99,6 +101,9 @@ _SIGS = {
 
 # The size of the no-allocation launch's static scratch array (EK_SCRATCH_BYTES).
 SCRATCH_BYTES = 16 << 20
+# The workspace of split launches (EK_WORKSPACE_BYTES), and its counters (one word a tile).
+WORKSPACE_BYTES = 16 << 20
+SPLIT_COUNTERS = 16384
 
 EXPORTED = sorted([*_SIGS, "ek_compile", "ek_buffer_free", "ek_version", "ek_runtime_version"])
 

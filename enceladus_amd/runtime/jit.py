@@ -173,10 +173,10 @@ _FMT = {"int32_t": ("i", 4), "int64_t": ("q", 8), "uint32_t": ("I", 4), "uint64_
 class _FastEntry:
     """A specialization's pre-packed launch: kernarg struct, function, block size."""
 
-    __slots__ = ("lc", "st", "fn", "block")
+    __slots__ = ("lc", "st", "fn", "block", "split")
 
-    def __init__(self, lc, st, fn, block):
-        self.lc, self.st, self.fn, self.block = lc, st, fn, block
+    def __init__(self, lc, st, fn, block, split):
+        self.lc, self.st, self.fn, self.block, self.split = lc, st, fn, block, split
 
 
 def _fast_entry(lc) -> "_FastEntry | None":
@@ -190,7 +190,7 @@ def _fast_entry(lc) -> "_FastEntry | None":
         fmt += "x" * pad + code
         off += pad + size
     fmt += "x" * ((-off) % 8)
-    return _FastEntry(lc, struct.Struct(fmt), lc.ck.function(), g.block)
+    return _FastEntry(lc, struct.Struct(fmt), lc.ck.function(), g.block, g.split)
 
 
 _tls = threading.local()
@@ -681,12 +681,20 @@ class JITFunction:
             return ent.lc.ck
         if _trace._active is not None:
             return None                 # `enceladus.capture` records the general path
+        if stream is None:
+            stream = _launch_stream()
+        if ent.split is not None:
+            ws, n = 0, 1
+            if gz == 1:
+                n = C.split_factor(ent.split, gx * gy, rt[ent.split["hi"]])
+                ws = C.workspace(stream) if n > 1 else 0
+            if ws:
+                gz = n
+            rt.append(ws)
         try:
             kb = ent.st.pack(*rt)
         except (struct.error, OverflowError):
             return None                 # a float beyond fp32's range: general packing
-        if stream is None:
-            stream = _launch_stream()
         t = _timing.current()
         if t is not None:
             t.launch(stream, ent.fn, (gx, gy, gz), ent.block, kb, len(kb))

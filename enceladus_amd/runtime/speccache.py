@@ -222,7 +222,7 @@ def _gen_to_json(gen) -> dict | None:
         return None
     return {"name": gen.name, "source": gen.source, "num_warps": gen.num_warps,
             "lds_bytes": gen.lds_bytes, "block": gen.block, "coarsen": gen.coarsen,
-            "asserts": asserts, "flush": flush,
+            "asserts": asserts, "flush": flush, "split": gen.split,
             "args": [[a.name, a.kind, a.dtype.name if a.dtype else None, a.cparam]
                      for a in gen.args]}
 
@@ -235,6 +235,7 @@ def _gen_from_json(d: dict):
     g.coarsen = d["coarsen"]
     g.asserts = d["asserts"]
     g.flush = d["flush"]
+    g.split = d["split"]
     g.report = None          # `explain` regenerates the report
     return g
 

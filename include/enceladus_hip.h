@@ -135,6 +135,19 @@ int ek_launch_flush_noalloc(void* stream, void* function, uint32_t gx, uint32_t 
                             size_t flush_scratch_offset, size_t scratch_bytes, char* err,
                             size_t errlen);
 
+/* No counterpart in the reference. The workspace of launches that split a k loop over several
+ * workgroups per tile (a float row per workgroup, after 16384 tile counters that are zero between
+ * launches): EK_WORKSPACE_BYTES of device memory kept for `stream` on the current device, made
+ * by the first call. Launches in one stream's order share it. Sets *ptr to NULL, and the caller
+ * launches without splitting, when the stream is being captured into a graph (replays on other
+ * streams would race on the workspace), when EK_WORKSPACES streams have one already, or when
+ * there is no memory. ek_stream_free gives a stream's workspace back; ek_workspace_release
+ * all of them, once their devices are idle (no split launch may be in preparation). */
+#define EK_WORKSPACE_BYTES (16u << 20)
+#define EK_WORKSPACES 8
+int ek_workspace(void* stream, void** ptr, char* err, size_t errlen);
+int ek_workspace_release(char* err, size_t errlen);
+
 /* Version string of the shim and of the HIP runtime it runs on. */
 const char* ek_version(void);
 int ek_runtime_version(int* version);

@@ -1,0 +1,115 @@
+"""Block GEMM loops split along k over several workgroups per tile: exact against integer
+products (every partial sum is exact), the same bits on every launch, whole against sliced, on
+several streams and threads, and under graph capture (where they do not split)."""
+
+import threading
+
+import numpy as np
+import pytest
+
+from enceladus_amd.runtime import compile as C
+from examples.matmul import matmul, matmul_desc
+from examples.matmul_fused import matmul_bias_gelu
+from tests.test_gpu_gemm_edges import whole
+
+pytestmark = pytest.mark.gpu
+
+
+def _force(monkeypatch, n):
+    monkeypatch.setattr(C, "split_factor", lambda split, tiles, hi: n)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "float32"])
+@pytest.mark.parametrize("slices", [1, 2, 3, 5, 16])
+@pytest.mark.parametrize("mnk", [(64, 64, 512), (1, 70, 500), (65, 130, 1000), (33, 9, 64)])
+def test_sliced_products_are_exact(mnk, slices, dtype, monkeypatch):
+    _force(monkeypatch, slices)
+    m, n, k = mnk
+    a, b = whole(m, k, 1, 0, dtype), whole(k, n, 2, 0, dtype)
+    want = (a.double() @ b.double()).cpu().numpy()
+    for f, tile in ((matmul_desc, (64, 64, 64)), (matmul, (64, 64, 32))):
+        for _ in range(3):           # the tile counters are back at zero after each launch
+            c = f(a, b, bm=tile[0], bn=tile[1], bk=tile[2])
+            assert np.array_equal(c.double().cpu().numpy(), want)
+
+
+def test_which_launches_split():
+    """Few tiles and a long k split; a grid that fills half of the CUs, or a short k, does not;
+    the slices' rows fit the workspace."""
+    from enceladus_amd.runtime import hip
+    cus = C.coarsen_cap()
+    sp = {"hi": 5, "bk": 64, "words": 4096, "step_us": 0.33}
+    assert C.split_factor(sp, 16, 8192) > 1
+    assert C.split_factor(sp, cus // 2 + 1, 1 << 20) == 1
+    assert C.split_factor(sp, 16, 512) == 1 and C.split_factor(sp, 16, 0) == 1
+    for tiles in (1, 3, 16, cus // 2):
+        for words in (1024, 16384, 65536):
+            for hi in (64, 4096, 1 << 24):
+                n = C.split_factor(dict(sp, words=words), tiles, hi)
+                assert n == 1 or (hip.SPLIT_COUNTERS + n * tiles * words) * 4 <= \
+                    hip.WORKSPACE_BYTES
+                assert n == 1 or n <= -(-hi // 64) // 2
+
+
+def test_epilogue_runs_once_and_is_deterministic(monkeypatch):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(0)
+    a = torch.randn(48, 2048, generator=g, device="cuda").half()
+    b = (torch.randn(2048, 200, generator=g, device="cuda") / 45).half()
+    bias = torch.randn(200, generator=g, device="cuda").half()
+    first = None
+    for n in (1, 4):
+        _force(monkeypatch, n)
+        outs = [matmul_bias_gelu(a, b, bias, bm=64, bn=64, bk=64) for _ in range(4)]
+        assert all(torch.equal(o, outs[0]) for o in outs)
+        first = outs[0] if first is None else first
+        torch.testing.assert_close(outs[0].float(), first.float(), rtol=2e-3, atol=1e-3)
+
+
+def test_streams_and_threads_have_their_own_workspace(monkeypatch):
+    import torch
+    _force(monkeypatch, 4)
+    a, b = whole(64, 4096, 1, 0), whole(4096, 128, 2, 0)
+    want = a.double() @ b.double()
+    bad = []
+
+    def work():
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(50):
+                c = matmul_desc(a, b, bm=64, bn=64, bk=64)
+            s.synchronize()
+            if not torch.equal(c.double(), want):
+                bad.append(1)
+    torch.cuda.synchronize()
+    ts = [threading.Thread(target=work) for _ in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
+
+
+def test_captured_launches_do_not_split(monkeypatch):
+    import torch
+    _force(monkeypatch, 4)
+    a, b = whole(64, 4096, 1, 0), whole(4096, 128, 2, 0)
+    c = torch.empty(64, 128, dtype=torch.float16, device="cuda")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        matmul_desc(a, b, c, bm=64, bn=64, bk=64)      # compiled and loaded before the capture
+    torch.cuda.synchronize()
+    want = c.clone()
+    g = torch.cuda.CUDAGraph()
+    seen = []
+    real = C.workspace
+    monkeypatch.setattr(C, "workspace", lambda st: seen.append(real(st)) or seen[-1])
+    with torch.cuda.graph(g, stream=s):
+        matmul_desc(a, b, c, bm=64, bn=64, bk=64)
+    assert seen == [0]
+    for _ in range(3):
+        c.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, want)
+        matmul_desc(a, b, bm=64, bn=64, bk=64)         # eager work between replays
