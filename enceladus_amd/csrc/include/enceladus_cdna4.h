@@ -365,6 +365,31 @@ template <int MASK, typename T> EK_INLINE T shfl_xor(T v) {
   }
 }
 
+// One step of a butterfly reduction over lanes: a and the value MASK lanes away combined, for
+// values that lanes differing only in the bits below MASK already share. Any lane of the other
+// group will then do, so 4 and 8 are one DPP mirror (lane ^ 7, lane ^ 15), which the compiler
+// folds into the operation, and 16 and 32 combine the two results of a swap as they are
+// (rows 0 and 1 for both, in the same order in every lane) instead of picking one by lane.
+template <typename OP, int MASK, typename T> EK_INLINE T reduce_xor(T v) {
+  if constexpr (sizeof(T) != 4) {
+    return OP::template op<T>(v, shfl_xor<MASK>(v));
+  } else {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    if constexpr (MASK >= 16) {
+      const auto r = [&] {
+        if constexpr (MASK == 16) return __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        else return __builtin_amdgcn_permlane32_swap(u, u, false, false);
+      }();
+      return OP::template op<T>(__builtin_bit_cast(T, (uint32_t)r[0]),
+                                __builtin_bit_cast(T, (uint32_t)r[1]));
+    } else {
+      constexpr int ctrl = MASK == 1 ? 0xB1 : MASK == 2 ? 0x4E : MASK == 4 ? 0x141 : 0x140;
+      return OP::template op<T>(v, __builtin_bit_cast(T, (uint32_t)__builtin_amdgcn_update_dpp(
+                                       0, (int)u, ctrl, 0xF, 0xF, true)));
+    }
+  }
+}
+
 // Inclusive prefix sum over lanes 0..63 of a 32-bit value with DPP moves: Kogge-Stone
 // inside each 16-lane row (row_shr 1, 2, 4, 8), then row_bcast:15 carries row 0 into
 // row 1 and row 2 into row 3, and row_bcast:31 carries lane 31 into rows 2 and 3. Lanes
