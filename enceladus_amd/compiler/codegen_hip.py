@@ -47,6 +47,18 @@ _INFIX = {"add": "+", "sub": "-", "mul": "*", "div": "/", "and": "&", "or": "|",
           "eq": "==", "ne": "!=", "lt": "<", "le": "<=", "gt": ">", "ge": ">="}
 
 
+def _feeds(op: ir.Op):
+    """Every value `op` is computed from, directly or through other ops."""
+    seen, todo = set(), list(op.operands)
+    while todo:
+        v = todo.pop()
+        if v.id not in seen:
+            seen.add(v.id)
+            yield v
+            if v.op is not None:
+                todo.extend(v.op.operands)
+
+
 def _through_trans(v: ir.Value) -> ir.Value:
     while v.op is not None and v.op.name == "trans":
         v = v.op.operands[0]
@@ -150,6 +162,7 @@ class GeneratedKernel:
     # indices), "total" (words per workgroup row of the partial buffer), "chunks" (64-word
     # column chunks)}; the launcher runs `name` on grid (chunks, rows / rb) after the kernel
     flush: dict | None = None
+    pack: int = 0          # programs (along grid x) per workgroup (0: one)
     # a block GEMM that may be split along k: {"hi" (index of the argument that bounds k), "bk",
     # "words" (floats of one workgroup's accumulator), "step_us" (a k step's time, roughly)}; its last argument is the workspace
     # (0: not split), and a split launch runs one workgroup per tile and slice (grid z)
@@ -192,6 +205,11 @@ class Emitter:
         self.fast_failed = False
         self.edge_only = False       # the general copy runs only for edge programs
         self.split: dict | None = None
+        self.pack = 0
+        self.assumed: set[str] = set()   # uniform conditions that hold where code is emitted
+        self.pid_expr: str | None = None  # the program id of the copy being emitted
+        # cyclic loads whose start is emitted already: (its name, whether the tile wraps)
+        self.cyclic_at: dict[int, tuple[str, bool]] = {}
 
     # ------------------------------------------------------------------ utilities
     def fresh(self, hint="v") -> str:
@@ -303,6 +321,16 @@ class Emitter:
             return None
         return base.op.operands[0], x, n.op.operands[0]
 
+    def _cyclic_start(self, x: ir.Value, n: ir.Value, ext: int) -> str:
+        """Emits `<q>x`, the first of the run x, and `<q>r`, its remainder by n; returns q. The
+        remainder is -1 for a run that is not of non-negative numbers, or a divisor that is
+        not positive."""
+        q, nn = self.fresh("cy"), self.name[n.id]
+        self.emit(f"const int {q}x = {self.cheap(x, ['0'])};")
+        self.emit(f"const int {q}r = {nn} > 0 && {q}x >= 0 && {q}x <= 0x7fffffff - {ext} ? "
+                  f"{q}x % {nn} : -1;")
+        return q
+
     def _cyclic_load(self, op, lay: LY.Layout, nm: str) -> bool:
         """An unmasked load through `base + x % n` without a division per element. The tile's
         first x % n is uniform; a tile that does not wrap is then one contiguous run, read like
@@ -319,26 +347,32 @@ class Emitter:
         t, ext = ctype(op.result.type.dtype), op.result.type.shape[0]
         b, nn = self.name[base.id], self.name[n.id]
         c = self.coord(lay, 0, "rv")
-        q = self.fresh("cy")
-        self.emit(f"const int {q}x = {self.cheap(x, ['0'])};")
-        # -1: not a run of non-negative numbers, or a divisor that is not positive
-        self.emit(f"const int {q}r = {nn} > 0 && {q}x >= 0 && {q}x <= 0x7fffffff - {ext} ? "
-                  f"{q}x % {nn} : -1;")
+        q, known = self.cyclic_at.get(id(op), (None, None))
+        q = q or self._cyclic_start(x, n, ext)
+
+        def run():
+            self._vec_loop(lay.nregs, V)
+            self.emit(f"  ek::vload_u<{t}, {V}>(&{nm}[rv], ({b} + {q}r) + (uint32_t)({c}));")
+            self.emit("}")
+
+        def wrapping():
+            self._vec_loop(lay.nregs, V)
+            self.emit(f"  const int ek_r = (int)((uint32_t)({q}x + {c}) % (uint32_t){nn});")
+            self.emit(f"  const int ek_s = ek_r - ek::Min::op<int>(ek_r, {nn} - {V});")
+            self.emit(f"  ek::vload_u<{t}, {V}>(&{nm}[rv], {b} + (ek_r - ek_s));")
+            self.emit("  if (__builtin_amdgcn_ballot_w64(ek_s > 0) != 0) {")
+            self.emit(f"    {t} ek_w[{V}];")
+            self.emit(f"    ek::vload_u<{t}, {V}>(ek_w, {b});")
+            self.emit(f"    ek::wrap_shift<{t}, {V}>(&{nm}[rv], ek_s, ek_w);")
+            self.emit("  }")
+            self.emit("}")
+        if known is not None:
+            wrapping() if known else run()
+            return True
         self.emit(f"if ({q}r >= 0 && {q}r <= {nn} - {ext}) {{")
-        self._vec_loop(lay.nregs, V)
-        self.emit(f"  ek::vload_u<{t}, {V}>(&{nm}[rv], ({b} + {q}r) + (uint32_t)({c}));")
-        self.emit("}")
+        run()
         self.emit(f"}} else if ({q}r >= 0 && {nn} >= {V}) {{")
-        self._vec_loop(lay.nregs, V)
-        self.emit(f"  const int ek_r = (int)((uint32_t)({q}x + {c}) % (uint32_t){nn});")
-        self.emit(f"  const int ek_s = ek_r - ek::Min::op<int>(ek_r, {nn} - {V});")
-        self.emit(f"  ek::vload_u<{t}, {V}>(&{nm}[rv], {b} + (ek_r - ek_s));")
-        self.emit("  if (__builtin_amdgcn_ballot_w64(ek_s > 0) != 0) {")
-        self.emit(f"    {t} ek_w[{V}];")
-        self.emit(f"    ek::vload_u<{t}, {V}>(ek_w, {b});")
-        self.emit(f"    ek::wrap_shift<{t}, {V}>(&{nm}[rv], ek_s, ek_w);")
-        self.emit("  }")
-        self.emit("}")
+        wrapping()
         self.emit("} else {")
         self.emit("#pragma unroll")
         self.emit(f"for (int r = 0; r < {lay.nregs}; ++r) {nm}[r] = *({self.elem(op.operands[0], lay, 'r')});")
@@ -1250,7 +1284,7 @@ class Emitter:
         nm = self.fresh("pid")
         ax = "xyz"[op.attrs["axis"]]
         src = f"ek_pid_{ax}" if (self.remap_pids or self.coarsen) else \
-            f"(int32_t)blockIdx.{ax}"
+            self.pid_expr or f"(int32_t)blockIdx.{ax}"
         self.emit(f"const int32_t {nm} = {src};")
         self.define(op.result, nm)
 
@@ -1394,6 +1428,10 @@ class Emitter:
         # Edge versioning: a mask that is provably all-true over a uniform runtime interval
         # (e.g. offs < n away from the last program) gets a branch-free unmasked path.
         cond = None if self.opt.get("no_edge_versioning") else self.all_true(mask)
+        if cond in self.assumed:
+            plain()
+            self.define(res, nm)
+            return
         if cond and self._assume(cond):
             if streaming and not self.opt.get("no_serial_streams"):
                 # One streaming tile load in flight per wave: waiting for the previous one
@@ -1680,7 +1718,7 @@ class Emitter:
         cond = None
         if mask is not None and not self.opt.get("no_edge_versioning"):
             cond = self.all_true(mask)
-        if cond and self._assume(cond):
+        if cond and (cond in self.assumed or self._assume(cond)):
             self._vec_loop(lay.nregs, V)
             open_vec()
             self.emit(f"  ek::{st}<{t}, {V}>({pe(0)}, &{at(0)});")
@@ -1917,6 +1955,106 @@ class Emitter:
             if op.regions or op.name in ("dot", "atomic_rmw", "atomic_cas", "assert", "print",
                                          "barrier", "desc_store"):
                 return False
+        return True
+
+    def _emit_packed(self, fn) -> bool:
+        """A flat program whose threads load less than 16 bytes at a time (1,024 16-bit elements
+        over 4 waves: 8) keeps too few bytes in flight to fill the memory pipes: its
+        workgroups then run `pack` programs each. Where all of them exist and are wholly
+        selected, their loads go out together and the rest of each follows (programs are
+        independent, so one's loads may pass another's stores); otherwise the workgroup runs
+        them one after the other. Straight-line 1-D elementwise programs on grid axis 0 only.
+        """
+        ops = fn.body.ops
+        loads = [o for o in ops if o.name == "load"]
+        stores = [o for o in ops if o.name == "store"]
+        if self.opt.get("no_pack") or not self._can_version(fn) or not loads or not stores or \
+                self.pid_axes != {0} or \
+                any(o.name not in ir.PURE_OPS | {"load", "store"} or
+                    o.name in ("num_programs", "join", "split", "shift", "reshape", "trans")
+                    for o in ops):
+            return False
+        nt, vec = self.nt, 0
+        for o in loads + stores:
+            p = o.operands[0]
+            if len(p.type.shape) != 1 or self.kind.get(p.id) != "cheap" or \
+                    p.type.numel % nt:
+                return False
+            run = self._cyclic(p) is not None or self.axis.get(p).contig[0] == p.type.shape[0]
+            if not run or p.type.numel != loads[0].result.type.numel:
+                return False
+            vec = max(vec, p.type.numel // nt * p.type.dtype.itemsize)
+        if not vec or vec >= 16 or any(
+                x.op is not None and x.op.name == "load" for o in loads for x in _feeds(o)):
+            return False
+        # to 16 bytes per thread and load (bf16 add of 2048 x 10240: 23.5 us with one program a
+        # workgroup, 20.3 with two, 20.4 with four)
+        self.pack = min(4, 16 // vec)
+        first = [o for o in ops if o.name in ir.PURE_OPS and not self.tile(o.result)
+                 and not any(x.op is not None and x.op.name == "load" for x in _feeds(o))]
+        rest = [o for o in ops if o not in first and o.name != "load"]
+        mark, lds = len(self.cur.items), self.lds
+        self.emit("{")
+        self.emit(f"const int ek_p0 = (int)blockIdx.x * {self.pack};")
+        conds, bound, good = [f"ek_p0 <= ek_np_x - {self.pack}"], [], True
+        runs, wraps = [], []
+        for u in range(self.pack):
+            self.pid_expr = f"(ek_p0 + {u})"
+            self.gen_block(fn.body, first)
+            at = {}
+            for o in loads + stores:
+                m = o.operands[1 if o.name == "load" else 2:]
+                if m:
+                    c = self.all_true(m[0])
+                    good = good and c is not None
+                    conds.append(c)
+                cyc = self._cyclic(o.operands[0])
+                if cyc is not None:
+                    good = good and o.name == "load"
+                    ext = o.operands[0].type.numel
+                    q = self._cyclic_start(cyc[1], cyc[2], ext)
+                    nn = self.name[cyc[2].id]
+                    runs.append(f"{q}r >= 0 && {q}r <= {nn} - {ext}")
+                    wraps.append(f"{q}r >= 0 && {nn} >= 16")
+                    at[id(o)] = q
+            bound.append(({r.id: self.name[r.id] for o in first for r in o.results
+                           if r.id in self.name}, at))
+        # with cyclic loads: one copy for tiles inside a period, one for tiles that wrap
+        for wrap, extra in enumerate((runs, wraps) if runs else ([],)):
+            if not good:
+                break
+            self.push_scope(f"if ({' && '.join(dict.fromkeys(conds + extra))}) {{")
+            self.assumed = set(conds)
+            made = []
+            for names, at in bound:
+                self.name.update(names)
+                self.cyclic_at = {k: (q, bool(wrap)) for k, q in at.items()}
+                self.gen_block(fn.body, loads)
+                made.append({o.result.id: self.name[o.result.id] for o in loads})
+            for (names, at), vals in zip(bound, made):
+                self.push_scope("{")
+                self.name.update(names)
+                self.name.update(vals)
+                self.gen_block(fn.body, rest)
+                self.pop_scope()
+                self.cur.memo.clear()
+            self.emit("return;")
+            self.pop_scope()
+        self.emit("}")
+        self.assumed, self.cyclic_at, self.pid_expr = set(), {}, None
+        self.fast_side = False
+        self.cur.memo.clear()
+        if not good or self.lds != lds:
+            del self.cur.items[mark:]
+            self.lds, self.pack = lds, 0
+            return False
+        self.push_scope(f"for (int ek_u = 0; ek_u < {self.pack}; ++ek_u) {{")
+        self.emit(f"const int ek_pid_x = (int)blockIdx.x * {self.pack} + ek_u;")
+        self.emit("if (ek_pid_x >= ek_np_x) break;")
+        self.pid_expr = "ek_pid_x"
+        self.gen_block(fn.body)
+        self.pid_expr = None
+        self.pop_scope()
         return True
 
     def all_true(self, m: ir.Value, depth=0):
@@ -3810,7 +3948,8 @@ class Emitter:
         # unmasked under a few uniform conditions (every program but the edge ones) runs a
         # fast copy without per-access branches and mask arithmetic; the first failing
         # guard jumps to the general copy before any store has run.
-        if self._can_version(fn):
+        packed = self._emit_packed(fn)
+        if not packed and self._can_version(fn):
             mark = len(self.scopes[0].items)
             report = {k: list(v) for k, v in self.report.items()}
             self.fast_mode = True
@@ -3827,7 +3966,8 @@ class Emitter:
                 self.scopes[0].items.append("    return;")
                 self.scopes[0].items.append("  " + "}" * (len(self.fast_conds) + 1))
                 self.edge_only = True
-        self.gen_block(fn.body)
+        if not packed:
+            self.gen_block(fn.body)
         kname = f"ek_{fn.name}"
         if self.asserts:
             params.append("uint32_t* ek_assert_buf")
@@ -3853,6 +3993,8 @@ class Emitter:
             args.append(KernelArg("ek_part", "ptr", core.int32, "int32_t*"))
         if self.coarsen:
             params += ["int32_t ek_np_x", "int32_t ek_np_y", "int32_t ek_np_z"]
+        elif self.pack:
+            params.append("int32_t ek_np_x")
         out = ['#include "enceladus_cdna4.h"', ""]
         attrs = f"__launch_bounds__({self.nt})"
         if getattr(self, "big_acc", 0) >= 128:
@@ -4009,6 +4151,7 @@ class Emitter:
         gk.asserts = list(self.asserts)
         gk.flush = flush
         gk.split = self.split
+        gk.pack = self.pack
         gk.report = self.report
         return gk
 

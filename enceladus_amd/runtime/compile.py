@@ -147,7 +147,7 @@ class CompiledKernel:
         values = list(values)
         if self.gen.flush or self.gen.split:
             values.append(0)      # the partial-bin buffer or workspace, set per stream at launch
-        b = codegen_hip.pack_args(self.args, values, pad8=not self.gen.coarsen)
+        b = codegen_hip.pack_args(self.args, values, pad8=not (self.gen.coarsen or self.gen.pack))
         self.packed_size = len(b)
         return b
 
@@ -248,6 +248,9 @@ class CompiledKernel:
     def launch_grid(self, grid):
         """(launch grid, extra kernarg bytes) for a logical program grid."""
         gx, gy, gz = (tuple(grid) + (1, 1, 1))[:3]
+        if self.gen.pack:
+            import struct
+            return (-(-gx // self.gen.pack), gy, gz), struct.pack("<i", gx)
         if not self.gen.coarsen:
             return (gx, gy, gz), b""
         total = gx * gy * gz

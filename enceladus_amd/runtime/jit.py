@@ -173,15 +173,15 @@ _FMT = {"int32_t": ("i", 4), "int64_t": ("q", 8), "uint32_t": ("I", 4), "uint64_
 
 class _FastEntry:
     """A specialization's pre-packed launch: kernarg struct, function, block size; how its k
-    loop may split; for a coarsened program walk, the workgroups its grid is capped at; for a
-    two-level flush, the second kernel's (function, kernarg struct, argument indices of the
+    loop may split; for a coarsened program walk, the workgroups its grid is capped at; the
+    programs each workgroup runs (0: one); for a two-level flush, the second kernel's (function, kernarg struct, argument indices of the
     flushed arrays, column chunks, rows per workgroup)."""
 
-    __slots__ = ("lc", "st", "fn", "block", "split", "cap", "flush")
+    __slots__ = ("lc", "st", "fn", "block", "split", "cap", "flush", "pack")
 
-    def __init__(self, lc, st, fn, block, split, cap, flush):
+    def __init__(self, lc, st, fn, block, split, cap, flush, pack):
         self.lc, self.st, self.fn, self.block = lc, st, fn, block
-        self.split, self.cap, self.flush = split, cap, flush
+        self.split, self.cap, self.flush, self.pack = split, cap, flush, pack
 
 
 def _fast_entry(lc) -> "_FastEntry | None":
@@ -200,12 +200,16 @@ def _fast_entry(lc) -> "_FastEntry | None":
         fmt += "x" * pad + "iii"
         off += pad + 12
         cap = max(1, C.coarsen_cap() * g.coarsen)
+    elif g.pack:
+        fmt += "x" * ((-off) % 4) + "i"
+        off += (-off) % 4 + 4
     fmt += "x" * ((-off) % 8)
     if g.flush:
         f = g.flush
         st = struct.Struct("<Qi4x" + "Q" * len(f["bases"]))
         flush = (lc.ck._flush_function(), st, tuple(f["bases"]), f["chunks"], f["rb"])
-    return _FastEntry(lc, struct.Struct(fmt), lc.ck.function(), g.block, g.split, cap, flush)
+    return _FastEntry(lc, struct.Struct(fmt), lc.ck.function(), g.block, g.split, cap, flush,
+                      g.pack)
 
 
 _tls = threading.local()
@@ -707,7 +711,10 @@ class JITFunction:
                 gz = n
             rt.append(ws)
         flush = ent.flush
-        if ent.cap:
+        if ent.pack:
+            rt.append(gx)
+            gx = -(-gx // ent.pack)
+        elif ent.cap:
             logical = (gx, gy, gz)
             gx, gy, gz = min(gx * gy * gz, ent.cap), 1, 1
             if flush is not None:

@@ -222,7 +222,7 @@ def _gen_to_json(gen) -> dict | None:
         return None
     return {"name": gen.name, "source": gen.source, "num_warps": gen.num_warps,
             "lds_bytes": gen.lds_bytes, "block": gen.block, "coarsen": gen.coarsen,
-            "asserts": asserts, "flush": flush, "split": gen.split,
+            "asserts": asserts, "flush": flush, "split": gen.split, "pack": gen.pack,
             "args": [[a.name, a.kind, a.dtype.name if a.dtype else None, a.cparam]
                      for a in gen.args]}
 
@@ -236,6 +236,7 @@ def _gen_from_json(d: dict):
     g.asserts = d["asserts"]
     g.flush = d["flush"]
     g.split = d["split"]
+    g.pack = d["pack"]
     g.report = None          # `explain` regenerates the report
     return g
 
