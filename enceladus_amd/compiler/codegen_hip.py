@@ -3590,6 +3590,18 @@ class Emitter:
         whole = rows and all(div(v) % 8 == 0 for v in (A["shape_v"][1], B["shape_v"][1]))
         buf = not (big or not whole or self.opt.get("no_buffer_loads"))
         bm, bn, bk = g["bm"], g["bn"], g["bk"]
+        kend = A["shape"][1]
+        if -(-(bm + bn) * bk * g["dt"].itemsize // 16 // self.nt) <= 2:
+            # Two of the program's k steps to one of the loop's, where a thread copies at most two
+            # chunks a step (64x64x32 on 4 waves: two MFMAs between barriers): the k slices run
+            # in the same order, so the bits are the same. What the program's last step does not
+            # cover must not come in with it: k ends with that step. bf16 at 64x64x32 on
+            # pointers: 1000 x 3000 x 2000 31.9 -> 30.6 us, 2048^3 38.3 -> 32.2; at 64x64x16
+            # 57.7 -> 37.6 and 48.7 -> 39.3. (128x128x32 is left alone: on descriptors 24.1 us
+            # as it is, 28.9 at 128x128x64, whose stages leave fewer workgroups to a CU.)
+            kend = (f"(int)ek::Min::op<int64_t>({kend}, {lo} + ((int64_t){hi} - {lo} + {bk - 1}) "
+                    f"/ {bk} * {bk})")
+            bk *= 2
         stage = (bm * bk + bk * bn) * g["dt"].itemsize
         dma = (buf and g["dt"] is not core.float32 and not self.opt.get("no_lds_dma") and (bm * bk // 8) % self.nt == 0
                and (bk * bn // 8) % self.nt == 0 and bn >= 32)
@@ -3633,7 +3645,7 @@ class Emitter:
             lo, hi = "ek_lo", "ek_hi"
         self.emit(f"  {tmpl} ek_g;")
         self.emit(f"  ek_g.run({nm}, {A['base']}, {A['strides'][0]}, {B['base']}, "
-                  f"{B['strides'][0]}, {A['shape'][0]}, {B['shape'][1]}, {A['shape'][1]}, "
+                  f"{B['strides'][0]}, {A['shape'][0]}, {B['shape'][1]}, {kend}, "
                   f"{self.name[g['m0'].id]}, {self.name[g['n0'].id]}, {lo}, {hi}, ek_smem, ek_tid);")
         if self.split:
             self.emit(f"  if (ek_ws && !ek::split_reduce<{lay.nregs}, {self.nt}>({nm}, ek_ws, "
