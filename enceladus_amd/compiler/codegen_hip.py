@@ -3597,8 +3597,8 @@ class Emitter:
             # in the same order, so the bits are the same. What the program's last step does not
             # cover must not come in with it: k ends with that step. bf16 at 64x64x32 on
             # pointers: 1000 x 3000 x 2000 31.9 -> 30.6 us, 2048^3 38.3 -> 32.2; at 64x64x16
-            # 57.7 -> 37.6 and 48.7 -> 39.3. (128x128x32 is left alone: on descriptors 24.1 us
-            # as it is, 28.9 at 128x128x64, whose stages leave fewer workgroups to a CU.)
+            # 57.7 -> 37.6 and 48.7 -> 39.3. (Four chunks a step, 128x128x32, is left alone: on
+            # aligned descriptors of 1000 x 3008 x 2000 24.1 us, where 128x128x64 takes 28.9.)
             kend = (f"(int)ek::Min::op<int64_t>({kend}, {lo} + ((int64_t){hi} - {lo} + {bk - 1}) "
                     f"/ {bk} * {bk})")
             bk *= 2
