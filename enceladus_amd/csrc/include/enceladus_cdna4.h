@@ -879,7 +879,9 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
 
   u32x4 r[PD][CH];
   // Of each chunk, from a k step's first column less EC (A: a chunk moved back from a ragged
-  // end starts up to EC - 1 columns before it) or first row (B).
+  // end starts up to EC - 1 columns before it) or first row (B), and there from the lowest of
+  // the operand's (A) or the step's (B) rows, which is the last one where rows descend (a
+  // negative row stride): 32-bit offsets are unsigned.
   Off off[CH], last[CH];    // of every k step, and of the last one
   int sh[CH], lsh[CH];      // elements to shift (EC and more: all zero), likewise
 
@@ -893,13 +895,15 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
     return B_TOT % NT == 0 || (i - A_CH) * NT + tid < B_TOT;
   }
 
-  EK_INLINE void plan(int lda, int ldb, int M, int N, int K, int m0, int n0, int klast, int tid) {
+  EK_INLINE void plan(int lda, int ldb, int M, int N, int K, int m0, int n0, int klast, Off low_a,
+                      Off low_b, int tid) {
 #pragma unroll
     for (int i = 0; i < A_CH; ++i) {
       const int row = m0 + row_a(i, tid), rc = Min::op<int>(row, M - 1), c = kc_a(i, tid) * EC;
       const int cl = Min::op<int>(klast + c, K - EC) - klast;    // 1 - EC and more
-      off[i] = ((Off)rc * (Off)lda + (Off)(c + EC)) * ES;
-      last[i] = ((Off)rc * (Off)lda + (Off)(cl + EC)) * ES;
+      const Off at = (Off)rc * (Off)lda - low_a;
+      off[i] = (at + (Off)(c + EC)) * ES;
+      last[i] = (at + (Off)(cl + EC)) * ES;
       sh[i] = row < M ? 0 : EC;
       lsh[i] = row < M ? c - cl : EC;
     }
@@ -907,8 +911,8 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
     for (int j = 0; j < B_CH; ++j) {
       const int i = A_CH + j, k = row_b(j, tid), gn = n0 + nc_b(j, tid) * EC;
       const int kl = Min::op<int>(klast + k, K - 1) - klast, nl = Min::op<int>(gn, N - EC);
-      off[i] = ((Off)k * (Off)ldb + (Off)nl) * ES;
-      last[i] = ((Off)kl * (Off)ldb + (Off)nl) * ES;
+      off[i] = ((Off)k * (Off)ldb - low_b + (Off)nl) * ES;
+      last[i] = ((Off)kl * (Off)ldb - low_b + (Off)nl) * ES;
       sh[i] = gn - nl;
       lsh[i] = kl == k ? gn - nl : EC;
     }
@@ -976,9 +980,11 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
     }
     const int klast = lo + (niter - 1) * BK;
     const bool edge = m0 + BM > M || n0 + BN > N, ragged = klast + BK > K;
-    plan(lda, ldb, M, N, K, m0, n0, klast, tid);
-    const char* a = reinterpret_cast<const char*>(A) + ((int64_t)lo - EC) * ES;
-    const char* b = reinterpret_cast<const char*>(B) + (int64_t)lo * ldb * ES;
+    const int64_t low_a = lda < 0 ? (int64_t)(M - 1) * lda : 0;
+    const int64_t low_b = ldb < 0 ? (int64_t)(Min::op<int>(BK, K) - 1) * ldb : 0;
+    plan(lda, ldb, M, N, K, m0, n0, klast, (Off)low_a, (Off)low_b, tid);
+    const char* a = reinterpret_cast<const char*>(A) + (low_a + lo - EC) * ES;
+    const char* b = reinterpret_cast<const char*>(B) + ((int64_t)lo * ldb + low_b) * ES;
     const int64_t sa = BK * ES, sb = (int64_t)BK * ldb * ES;
 #pragma unroll
     for (int p = 0; p < PD; ++p) {

@@ -86,3 +86,16 @@ def test_broadcast_operands_through_the_wrapper():
     y = torch.randint(-3, 4, (1, n)).half().cuda()
     a = torch.randint(-3, 4, (m, k)).half().cuda()
     assert torch.equal(matmul(a, y.expand(k, n)).double(), a.double() @ y.double().expand(k, n))
+
+
+@pytest.mark.parametrize("dtype", ["float16", "float32"])
+@pytest.mark.parametrize("mnk", SIZES)
+def test_descending_rows(mnk, dtype):
+    """A pointer to the last row in memory and a negative stride (32-bit offsets are unsigned)."""
+    m, n, k = mnk
+    for tile in TILES[:2]:
+        for sa in (-k, -(k + 24), -16, -3):
+            check(mnk, tile, sa, n, dtype)
+        for sb in (-n, -(n + 24), -16, -3):
+            check(mnk, tile, k, sb, dtype)
+        check(mnk, tile, -k, -(n + 8), dtype)
