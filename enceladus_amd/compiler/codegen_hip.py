@@ -3580,14 +3580,16 @@ class Emitter:
         p = g["plan"]
         T = ctype(g["dt"])
         A, B = g["A"], g["B"]
-        # LDS DMA needs rows of whole 16-byte chunks (bases, strides, K and N known to be
-        # multiples of 8 elements: a chunk is then wholly inside its row or out of range) and
-        # 32-bit byte offsets; anything else goes through registers (ek::GemmReg).
+        # LDS DMA needs rows of whole 16-byte chunks (bases, strides, K and N, the first k and the
+        # tile's first column known to be multiples of 8 elements: a chunk is then wholly
+        # inside its row or out of range) and 32-bit byte offsets; anything else goes through
+        # registers (ek::GemmReg).
         div = lambda v: self.axis.get(v).div[0]  # noqa: E731
         big = any(v.facts.get("span2g") for v in (A["base_v"], B["base_v"]))
         rows = all(div(v) >= 16 for v in (A["base_v"], B["base_v"])) and \
             all(div(v) % 8 == 0 for v in (A["stride_v"][0], B["stride_v"][0]))
-        whole = rows and all(div(v) % 8 == 0 for v in (A["shape_v"][1], B["shape_v"][1]))
+        whole = rows and all(div(v) % 8 == 0 for v in (A["shape_v"][1], B["shape_v"][1],
+                                                       op.operands[0], g["n0"]))
         buf = not (big or not whole or self.opt.get("no_buffer_loads"))
         bm, bn, bk = g["bm"], g["bn"], g["bk"]
         kend = A["shape"][1]

@@ -78,3 +78,61 @@ def test_steps_of_a_short_tile_cover_no_more_of_k(span, bk, dtype, k):
     c = torch.full((m, n), -1.0, device="cuda")
     part_of_k[(2, 2)](a, b, c, m, n, k, first, last, BM=64, BN=64, BK=bk, num_warps=4)
     assert torch.equal(c.double(), want)
+
+
+@pytest.mark.parametrize("bk", [16, 32, 64])
+@pytest.mark.parametrize("first,dma", [(0, True), (16, True), (48, True), (5, False), (8, False),
+                                       (12, False)])
+def test_k_ranges_of_aligned_operands(first, dma, bk):
+    """LDS DMA moves whole 16-byte chunks: only ranges that start on one take it, and their
+    merged steps cover no more of k than the program's (NaN beyond); the last elements stay."""
+    import torch
+    m, n, k = 96, 80, 208
+    for last in (first + 1, 100, 160, 207, 208, 300):
+        end = min(k, first + -(-max(last - first, 0) // bk) * bk)
+        a, b = whole(m, k, 1, 0), whole(k, n, 2, 0)
+        want = a[:, first:end].double() @ b[first:end].double()
+        a[:, end:], b[end:], a[:, :first], b[:first] = (float("nan"),) * 4
+        c = torch.full((m, n), -1.0, device="cuda")
+        ck = part_of_k[(2, 2)](a, b, c, m, n, k, first, last, BM=64, BN=64, BK=bk, num_warps=4)
+        assert ("ek::GemmDma" in ck.hip) == dma
+        assert torch.equal(c.double(), want), (first, last)
+
+
+@ek.jit
+def shifted_columns(a_ptr, b_ptr, c_ptr, M, N, K, BY: tl.constexpr, POINTERS: tl.constexpr,
+                    BM: tl.constexpr, BN: tl.constexpr, BK: tl.constexpr):
+    m0 = tl.program_id(0) * BM
+    n0 = tl.program_id(1) * BN + BY
+    rm, rn, rk = m0 + tl.arange(0, BM), n0 + tl.arange(0, BN), tl.arange(0, BK)
+    acc = tl.zeros((BM, BN), dtype=tl.float32)
+    if POINTERS:
+        ap = a_ptr + rm[:, None] * K + rk[None, :]
+        bp = b_ptr + rk[:, None] * N + rn[None, :]
+        for k in range(0, K, BK):
+            a = tl.load(ap, mask=(rm[:, None] < M) & (rk[None, :] + k < K), other=0.0)
+            b = tl.load(bp, mask=(rk[:, None] + k < K) & (rn[None, :] < N), other=0.0)
+            acc = tl.dot(a, b, acc)
+            ap += BK
+            bp += BK * N
+    else:
+        da = tl.make_tensor_descriptor(a_ptr, [M, K], [K, 1], [BM, BK])
+        db = tl.make_tensor_descriptor(b_ptr, [K, N], [N, 1], [BK, BN])
+        for k in range(0, K, BK):
+            acc = tl.dot(da.load([m0, k]), db.load([k, n0]), acc)
+    tl.store(c_ptr + rm[:, None] * N + rn[None, :], acc,
+             mask=(rm[:, None] < M) & (rn[None, :] < N))
+
+
+@pytest.mark.parametrize("pointers", [False, True])
+@pytest.mark.parametrize("by", [0, 3, 4, 8])
+def test_tiles_whose_first_column_starts_no_chunk(by, pointers):
+    import torch
+    m, n, k = 64, 176, 96
+    a, b = whole(m, k, 1, 0), whole(k, n, 2, 0)
+    c = torch.full((m, n), -1.0, device="cuda")
+    ck = shifted_columns[(1, 3)](a, b, c, m, n, k, BY=by, POINTERS=pointers, BM=64, BN=64, BK=32,
+                                 num_warps=4)
+    assert ("ek::GemmDma" in ck.hip) == (by % 8 == 0) and "ek::Gemm" in ck.hip
+    assert torch.equal(c[:, by:].double(), (a.double() @ b.double())[:, by:])
+    assert bool((c[:, :by] == -1).all())
