@@ -1963,7 +1963,9 @@ class Emitter:
         workgroups then run `pack` programs each. Where all of them exist and are wholly
         selected, their loads go out together and the rest of each follows (programs are
         independent, so one's loads may pass another's stores); otherwise the workgroup runs
-        them one after the other. Straight-line 1-D elementwise programs on grid axis 0 only.
+        them one after the other. Straight-line 1-D elementwise programs on grid axis 0 only,
+        and only those that load everything before they store: a later load may read what
+        its own program stored, through the same argument or another one of the same array.
         """
         ops = fn.body.ops
         loads = [o for o in ops if o.name == "load"]
@@ -1972,7 +1974,7 @@ class Emitter:
                 self.pid_axes != {0} or \
                 any(o.name not in ir.PURE_OPS | {"load", "store"} or
                     o.name in ("num_programs", "join", "split", "shift", "reshape", "trans")
-                    for o in ops):
+                    for o in ops) or ops.index(loads[-1]) > ops.index(stores[0]):
             return False
         nt, vec = self.nt, 0
         for o in loads + stores:

@@ -89,3 +89,33 @@ def test_other_launch_paths(tmp_path):
 def test_programs_that_reduce_stay_unpacked():
     x = np.zeros(2048, np.float16)
     assert "ek_np_x" not in _reduce_rows.warmup(x, x, 2048, BLOCK=1024).hip
+
+
+@enceladus.jit
+def _reads_back(p_ptr, q_ptr, o_ptr, n, BLOCK: tl.constexpr):
+    i = tl.program_id(0) * BLOCK + tl.arange(0, BLOCK)
+    m = i < n
+    x = tl.load(p_ptr + i, mask=m)
+    tl.store(p_ptr + i, x + x, mask=m)
+    y = tl.load(q_ptr + i, mask=m)
+    tl.store(o_ptr + i, y + y, mask=m)
+
+
+@pytest.mark.parametrize("dtype", ["int8", "float16"])
+@pytest.mark.parametrize("aliased", [False, True])
+@pytest.mark.parametrize("n", [1024, 2048, 5000])
+def test_programs_that_read_what_they_stored(n, aliased, dtype):
+    """Loads stay behind the stores before them, through the same or another argument."""
+    import torch
+    p = torch.arange(n).remainder(15).to(getattr(torch, dtype)).cuda()
+    q = p if aliased else p + 1
+    o = torch.zeros_like(p)
+    want_o = 4 * p if aliased else 2 * q
+    want_p = 2 * p
+    _reads_back[(enceladus.cdiv(n, 1024),)](p, q, o, n, BLOCK=1024)
+    assert torch.equal(p, want_p) and torch.equal(o, want_o)
+
+
+def test_programs_that_load_after_a_store_stay_unpacked():
+    x = np.zeros(2048, np.float16)
+    assert "ek_np_x" not in _reads_back.warmup(x, x, x, 2048, BLOCK=1024).hip
