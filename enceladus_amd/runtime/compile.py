@@ -350,7 +350,8 @@ def build_module(jfn, arg_types, arg_facts, constexprs, num_warps, options) -> i
     if not (options or {}).get("no_simplify"):
         simplify.simplify(fn)
         verify.maybe_verify(fn, "the simplifier")
-    if not (options or {}).get("no_pointer_gemm") and pointer_gemm.lift_pointer_gemm(fn):
+    lifted = not (options or {}).get("no_pointer_gemm") and pointer_gemm.lift_pointer_gemm(fn)
+    if lifted:
         verify.maybe_verify(fn, "the pointer matmul rewrite")
         ir.dce(fn)
     if widen.needs_idx64(fn):
@@ -361,4 +362,9 @@ def build_module(jfn, arg_types, arg_facts, constexprs, num_warps, options) -> i
         verify.maybe_verify(fn, "the attention scale rewrite")
     ir.dce(fn)
     verify.maybe_verify(fn, "dead-code elimination")
+    if lifted and codegen_hip.generate(fn, options).lds_bytes > codegen_hip.MAX_LDS:
+        # Two LDS stages of such tiles do not fit (fp16 256x128x128): the loop as written
+        # needs LDS for one tile at a time, in passes where that does not fit either.
+        return build_module(jfn, arg_types, arg_facts, constexprs, num_warps,
+                            {**(options or {}), "no_pointer_gemm": True})
     return fn

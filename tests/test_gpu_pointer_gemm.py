@@ -46,3 +46,14 @@ def test_lifted_loops_match_the_general_lowering(kind, mnk, monkeypatch):
                     BN=64, BK=32)
         outs.append(c.cpu())
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("tile", [(256, 128, 128, 8), (32, 128, 256, 8), (256, 256, 128, 8),
+                                  (64, 64, 256, 8)])
+@pytest.mark.parametrize("mnk", [(130, 257, 200), (256, 128, 512)])
+def test_tiles_with_and_without_room_for_two_stages(mnk, tile):
+    m, n, k = mnk
+    a, b = whole(m, k, 1, 0), whole(k, n, 2, 0)
+    bm, bn, bk, nw = tile
+    c = matmul(a, b, bm=bm, bn=bn, bk=bk, num_warps=nw)
+    assert np.array_equal(c.double().cpu().numpy(), (a.double() @ b.double()).cpu().numpy())

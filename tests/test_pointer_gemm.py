@@ -87,3 +87,27 @@ def test_strided_k_and_small_tiles_stay():
     assert "desc_load" in _ops("plain", dtype=np.zeros(16, np.float32))
     assert "desc_load" not in _ops("plain", sk=2)
     assert "desc_load" not in _ops("plain", bm=16)
+
+
+@pytest.mark.parametrize("tile", [(256, 128, 128, 8), (128, 64, 256, 4), (32, 128, 256, 8),
+                                  (64, 256, 256, 8), (256, 256, 128, 8)])
+@pytest.mark.parametrize("mnk", [(1000, 3000, 2000), (1024, 1024, 1024)])
+def test_tiles_whose_stages_do_not_fit_stay(tile, mnk):
+    """Two LDS stages of these tiles are past 160 KB: the loops keep their pointer loads and
+    compile, as they do without the rewrite."""
+    from examples.matmul import matmul_kernel
+    (bm, bn, bk, nw), (m, n, k) = tile, mnk
+    args = (H, H, H, m, n, k, k, 1, n, 1, n, 1)
+    meta = dict(BM=bm, BN=bn, BK=bk, num_warps=nw)
+    names = [op.name for op in ir.walk(matmul_kernel.ir(*args, **meta).body)]
+    assert "desc_load" not in names and names.count("load") == 2
+    assert matmul_kernel.warmup(*args, **meta).lds_bytes <= 160 * 1024
+
+
+def test_tiles_whose_stages_fit_are_lifted():
+    from examples.matmul import matmul_kernel
+    for bm, bn, bk, nw in ((64, 64, 256, 8), (256, 256, 64, 8), (128, 128, 128, 4)):
+        names = [op.name for op in ir.walk(matmul_kernel.ir(
+            H, H, H, 1000, 3000, 2000, 2000, 1, 3000, 1, 3000, 1, BM=bm, BN=bn, BK=bk,
+            num_warps=nw).body)]
+        assert names.count("desc_load") == 2
