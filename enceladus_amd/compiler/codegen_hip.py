@@ -1089,7 +1089,11 @@ class Emitter:
         # the image's slowest dim has the pass number in its top bits
         shape, k = list(a.shape), 0
         strides, total = self.lds_addr(shape, order, es)
+        whole = total * es
         while total * es > MAX_LDS:
+            if shape[order[-1]] == 1:
+                raise CompilationError(f"a layout conversion of a {a.shape} tile needs {whole} "
+                                       "bytes of LDS")
             shape[order[-1]] //= 2
             k += 1
             strides, total = self.lds_addr(shape, order, es)

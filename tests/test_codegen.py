@@ -516,3 +516,26 @@ def test_split_sink_keeps_source_order_around_a_store():
     assert len(parts) == 3, "expected the split-stage loop (two barriers)"
     assert "ek::exp2_fast(__builtin_fmaf(" in parts[1] and "ek::cvt<ek::bf16>" in parts[1]
     assert "ek::exp2_fast(" not in parts[2]
+
+
+@enceladus.jit
+def _cumsum_transposed(x_ptr, o_ptr, R: tl.constexpr, C: tl.constexpr):
+    r, c = tl.arange(0, R)[:, None], tl.arange(0, C)[None, :]
+    y = tl.cumsum(tl.load(x_ptr + c * R + r), axis=1)
+    tl.store(o_ptr + r * C + c, y)
+
+
+@pytest.mark.parametrize("shape", [(2, 65536), (4, 65536)])
+def test_conversions_no_slice_of_which_fits_are_refused(shape):
+    """Passes halve the image's slowest dimension; a tile one slice of which is past the LDS
+    is a clear error, not an image without memory."""
+    x = np.zeros(16, np.float32)
+    with pytest.raises(enceladus.CompilationError, match="layout conversion .* bytes of LDS"):
+        _cumsum_transposed.warmup(x, x, R=shape[0], C=shape[1], num_warps=8)
+
+
+@pytest.mark.parametrize("shape", [(2, 16384), (4, 16384), (16, 4096), (64, 1024)])
+def test_conversions_in_passes_stay_within_the_lds(shape):
+    x = np.zeros(16, np.float32)
+    ck = _cumsum_transposed.warmup(x, x, R=shape[0], C=shape[1], num_warps=8)
+    assert ck.lds_bytes <= codegen_hip.MAX_LDS and ">> -" not in ck.hip

@@ -338,3 +338,14 @@ def test_associative_scan(case, dtype, m, n, ax, rev, nw):
     if case == "add" and dtype is np.int32:
         ref = np.flip(np.cumsum(np.flip(x, ax), axis=ax), ax) if rev else np.cumsum(x, axis=ax)
         np.testing.assert_array_equal(out.reshape(m, n), ref.astype(dtype))
+
+
+@pytest.mark.parametrize("shape", [(2, 16384), (4, 16384), (16, 4096), (64, 1024)])
+def test_conversions_in_passes(shape):
+    """Tiles whose image fits the LDS at once, in two slices, or in more."""
+    from tests.test_codegen import _cumsum_transposed
+    r, c = shape
+    x = np.random.default_rng(0).integers(-9, 9, (c, r)).astype(np.float32)
+    out = np.zeros((r, c), np.float32)
+    _cumsum_transposed[(1,)](x, out, R=r, C=c, num_warps=8)
+    assert np.array_equal(out, np.cumsum(x.T, axis=1))
