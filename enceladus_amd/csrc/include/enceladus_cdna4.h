@@ -268,7 +268,7 @@ template <typename T, int V> EK_INLINE void edge_shift(T* v, int s, const T* o) 
     __builtin_memcpy(&x, v, sizeof(U));
     __builtin_memcpy(&f, o, sizeof(U));
     const int n = B * (s & (V - 1));
-    const U sel = (U)(~(U)0 >> n);            // the V - s elements that were read
+    const U sel = (U)((U)~(U)0 >> n);         // the V - s elements that were read
     x = (U)((x >> n) & sel) | (U)(f & (U)~sel);
     __builtin_memcpy(v, &x, sizeof(U));
   }
