@@ -27,11 +27,11 @@ the program's scalar values. A load qualifies when
 - its mask is a conjunction of upper bounds `i_d + offset < bound`, the one along k shrinking by
   the block's extent per step, and its `other` is zero (no mask: everything is selected).
 
-A tile whose origin is a program id times a constant becomes an offset into the whole operand;
-any other one gets a descriptor based at its own first element, whose shape is the number of rows
-(A) or columns (B) the mask selects, so the rewritten loop reads exactly the selected elements
-whatever the sign of the offsets. Kernels with arrays past 2^31 elements (64-bit index math) are left
-alone, as descriptors cannot address them.
+A tile whose origin is a program id times a constant, counted from one base for all of them,
+becomes an offset into the whole operand; any other one gets a descriptor based at its own first
+element, whose shape is the number of rows (A) or columns (B) the mask selects, so the rewritten
+loop reads exactly the selected elements whatever the sign of the offsets. Kernels with arrays
+past 2^31 elements (64-bit index math) are left alone, as descriptors cannot address them.
 """
 
 from __future__ import annotations
@@ -221,7 +221,7 @@ class _Loop:
     """One candidate loop, its analysis and its rewrite."""
 
     def __init__(self, fn: ir.Func, block: ir.Block, op: ir.Op, uses: dict):
-        self.block, self.op, self.uses = block, op, uses
+        self.fn, self.block, self.op, self.uses = fn, block, op, uses
         self.body = op.regions[0]
         self.iv = self.body.args[0]
         self.an = _Analysis()
@@ -403,6 +403,26 @@ class _Loop:
                                  ("program_id", "num_programs") for a in k)
                    for k, c in p.t.items())
 
+    def same_base(self, base: ir.Value, rest: _Poly, first: _Poly) -> bool:
+        """Whether programs that differ only in the program ids of `first` address their tiles
+        from one place: the base is an argument, and nothing in `rest`, the offset less the
+        tile's origin, depends on those ids (nor on a value whose origin is not in sight).
+        Operands stored tile by tile, or behind a pointer per tile, fail this: the rows
+        and columns before such a tile are not the operand's."""
+        pids = {self.an.atom[a].op.attrs.get("axis", 0) for a in first.atoms()
+                if self.an.atom[a].op.name == "program_id"}
+        todo, seen = [base, *(self.an.atom[a] for a in rest.atoms())], set()
+        while todo:
+            v = todo.pop()
+            if v.id in seen or v in self.fn.args:
+                continue
+            seen.add(v.id)
+            if v.op is None or v.op.regions or \
+                    (v.op.name == "program_id" and v.op.attrs.get("axis", 0) in pids):
+                return False
+            todo.extend(v.op.operands)
+        return True
+
     def extent(self, bounds, most: int) -> ir.Value:
         """min(most, limits), at least 0: how many leading coordinates are selected. Computed
         in 64 bits, where `limit - offset` cannot wrap."""
@@ -458,20 +478,23 @@ class _Loop:
             shape[kd] = self.k_extent(p["bounds"][kd], hi)
             offs[kd] = self.iv
             first = p["bounds"][od][0][1] if p["bounds"][od] else None
-            if first is not None and self.from_pids(first) and \
-                    all(b[1] == first for b in p["bounds"][od]):
+            rest = None if first is None else \
+                off - first * (p["stride"] if od == 0 else _Poly.const(1))
+            if rest is not None and self.from_pids(first) and \
+                    all(b[1] == first for b in p["bounds"][od]) and \
+                    self.same_base(base, rest, first):
                 # a tile at `first` = program id x tile size, never before the operand: the
                 # whole operand is described and the tile's origin is an offset into it
                 offs[od] = self.poly(first)
-                off = off - first * (p["stride"] if od == 0 else _Poly.const(1))
+                off = rest
                 shape[od] = self.k_extent([(lim, _Poly(), extra) for lim, _, extra in
                                            p["bounds"][od]], None)
             else:
                 shape[od] = self.extent(p["bounds"][od], p["shape"][od])
             if off.value() != 0:
                 base = self.emit("ptr_add", [base, self.poly(off)], [base.type])
-            if root.facts.get("span2g"):
-                base.facts["span2g"] = True
+            if root not in self.fn.args or root.facts.get("span2g"):
+                base.facts["span2g"] = True       # (a base of unknown origin may span as much)
             strides = [self.poly(p["stride"]), self.iconst(1)]
             d = self.emit("make_desc", [base, *shape, *strides],
                           [ir.DescType(p["dtype"], tuple(p["shape"]))])

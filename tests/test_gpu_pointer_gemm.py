@@ -7,7 +7,7 @@ import pytest
 import enceladus
 from examples.matmul import matmul
 from tests.test_gpu_gemm_edges import whole
-from tests.test_pointer_gemm import KEPT, LIFTED, _loop
+from tests.test_pointer_gemm import KEPT, LIFTED, _loop, _stored_by_tile
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +57,24 @@ def test_tiles_with_and_without_room_for_two_stages(mnk, tile):
     bm, bn, bk, nw = tile
     c = matmul(a, b, bm=bm, bn=bn, bk=bk, num_warps=nw)
     assert np.array_equal(c.double().cpu().numpy(), (a.double() @ b.double()).cpu().numpy())
+
+
+@pytest.mark.parametrize("kind", ["blocks", "table"])
+@pytest.mark.parametrize("mnk", [(100, 90, 70), (64, 128, 96), (70, 131, 33), (5, 3, 64)])
+def test_operands_stored_by_tile(kind, mnk):
+    """Blocks of columns one after the other, with surplus programs past the last one."""
+    import torch
+    m, n, k = mnk
+    bn = 64
+    nb = enceladus.cdiv(n, bn)
+    a, b = whole(m, k, 1, 0), whole(k, n, 2, 0)
+    at = torch.arange(nb).flip(0) if kind == "table" else torch.arange(nb)
+    blocks = torch.full((nb, k, bn), float("nan"), dtype=torch.float16, device="cuda")
+    for i in range(nb):
+        cols = b[:, i * bn:(i + 1) * bn]
+        blocks[at[i], :, :cols.shape[1]] = cols
+    table = (at * k * bn).to(torch.int32).cuda()
+    c = torch.full((m, n), 7.0, device="cuda")
+    _stored_by_tile[(nb + 2, enceladus.cdiv(m, 64) + 1)](
+        a, blocks, c, table, m, n, k, k, KIND=kind, BM=64, BN=bn, BK=32)
+    assert torch.equal(c.double(), a.double() @ b.double())

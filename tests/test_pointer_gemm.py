@@ -111,3 +111,39 @@ def test_tiles_whose_stages_fit_are_lifted():
             H, H, H, 1000, 3000, 2000, 2000, 1, 3000, 1, 3000, 1, BM=bm, BN=bn, BK=bk,
             num_warps=nw).body)]
         assert names.count("desc_load") == 2
+
+
+@enceladus.jit
+def _stored_by_tile(a_ptr, b_ptr, c_ptr, t_ptr, M, N, K, sa, KIND: tl.constexpr,
+                    BM: tl.constexpr, BN: tl.constexpr, BK: tl.constexpr):
+    """B in blocks of BN columns, [K, BN] each, one after the other, or at places of a table."""
+    pn, pm = tl.program_id(0), tl.program_id(1)
+    rm, rk, cn = pm * BM + tl.arange(0, BM), tl.arange(0, BK), tl.arange(0, BN)
+    ap = a_ptr + rm[:, None] * sa + rk[None, :]
+    at = pn * (K * BN)
+    if KIND == "table":
+        at = tl.load(t_ptr + pn, mask=pn * BN < N, other=0)
+    bp = b_ptr + at + rk[:, None] * BN + cn[None, :]
+    acc = tl.zeros((BM, BN), dtype=tl.float32)
+    for k in range(0, K, BK):
+        a = tl.load(ap, mask=(rm[:, None] < M) & (rk[None, :] + k < K), other=0.0)
+        b = tl.load(bp, mask=(rk[:, None] + k < K) & ((pn * BN + cn)[None, :] < N), other=0.0)
+        acc = tl.dot(a, b, acc)
+        ap += BK
+        bp += BK * BN
+    rn = pn * BN + cn
+    tl.store(c_ptr + rm[:, None] * N + rn[None, :], acc,
+             mask=(rm[:, None] < M) & (rn[None, :] < N))
+
+
+@pytest.mark.parametrize("kind", ["blocks", "table"])
+def test_operands_stored_by_tile_are_described_tile_by_tile(kind):
+    """Only what a program's own mask selects belongs to its tile: its descriptor starts at the
+    tile (column 0) and ends with the selected columns, unlike A's, which is the whole operand."""
+    f = _stored_by_tile.ir(H, H, np.zeros(4, np.float32), np.zeros(4, np.int32), 100, 90, 70, 70,
+                           KIND=kind, BM=64, BN=64, BK=32)
+    loads = [op for op in ir.walk(f.body) if op.name == "desc_load"]
+    assert len(loads) == 2
+    a, b = loads
+    assert b.operands[2].op.name == "const" and b.operands[2].op.attrs["value"] == 0
+    assert a.operands[1].op.name != "const"
