@@ -164,8 +164,10 @@ class GeneratedKernel:
     flush: dict | None = None
     pack: int = 0          # programs (along grid x) per workgroup (0: one)
     # a block GEMM that may be split along k: {"hi" (index of the argument that bounds k), "bk",
-    # "words" (floats of one workgroup's accumulator), "step_us" (a k step's time, roughly)}; its last argument is the workspace
-    # (0: not split), and a split launch runs one workgroup per tile and slice (grid z)
+    # "words" (floats of one workgroup's accumulator), "step_us" (a k step's time, roughly),
+    # "serial" (the function for launches without a workspace)}; its last arguments are the
+    # workspace (0: not split) and the number of slices, and a split launch runs one workgroup per
+    # tile and slice (grid z), or the serial function with one workgroup per tile
     split: dict | None = None
     # what `kernel.explain` reports: {"conversions", "lds", "dots"} recorded by the emitter
     report: dict = field(default_factory=dict)
@@ -3636,28 +3638,40 @@ class Emitter:
             # MB (64x64x128 fp16: 0.65 us measured), or its MFMAs at half their peak
             # (128x128x64 fp32: 5.2 us)
             rate = 0.4e6 if g["dt"] is core.float32 else 4.9e6
-            self.split = {"hi": next(i for i, a in enumerate(self.fn.args)
+            self.split = {"serial": f"ek_{self.fn.name}_serial", "hi": next(i for i, a in enumerate(self.fn.args)
                                      if a is op.operands[1]), "bk": bk,
                           "words": lay.nregs * self.nt,
                           "step_us": round(max(2e-5 * stage, 2 * bm * bn * bk / rate), 3)}
-            self.emit(f"  int ek_lo = {lo}, ek_hi = {hi};")
-            self.emit("  if (ek_ws) {")
-            self.emit(f"    const int ek_per = ek::split_slice(ek_lo, ek_hi, {bk}, gridDim.z);")
-            self.emit("    ek_lo += (int)blockIdx.z * ek_per;")
-            self.emit("    ek_hi = ek::Min::op<int>(ek_hi, ek_lo + ek_per);")
-            self.emit("    if (blockIdx.z) {")
-            self.emit("      #pragma unroll")
-            self.emit(f"      for (int r = 0; r < {lay.nregs}; ++r) {nm}[r] = 0.0f;")
-            self.emit("    }")
-            self.emit("  }")
-            lo, hi = "ek_lo", "ek_hi"
+        run = (f"  ek_g.run({nm}, {A['base']}, {A['strides'][0]}, {B['base']}, "
+               f"{B['strides'][0]}, {A['shape'][0]}, {B['shape'][1]}, {kend}, "
+               f"{self.name[g['m0'].id]}, {self.name[g['n0'].id]}, ")
         self.emit(f"  {tmpl} ek_g;")
-        self.emit(f"  ek_g.run({nm}, {A['base']}, {A['strides'][0]}, {B['base']}, "
-                  f"{B['strides'][0]}, {A['shape'][0]}, {B['shape'][1]}, {kend}, "
-                  f"{self.name[g['m0'].id]}, {self.name[g['n0'].id]}, {lo}, {hi}, ek_smem, ek_tid);")
-        if self.split:
-            self.emit(f"  if (ek_ws && !ek::split_reduce<{lay.nregs}, {self.nt}>({nm}, ek_ws, "
-                      "ek_smem, ek_tid)) return;")
+        if not self.split:
+            self.emit(f"{run}{lo}, {hi}, ek_smem, ek_tid);")
+        else:
+            n = lay.nregs
+            ind = self.cur.indent
+            parallel = [
+                f"  int ek_lo = {lo}, ek_hi = {hi};",
+                "  if (ek_ws) {",
+                f"    const int ek_per = ek::split_slice(ek_lo, ek_hi, {bk}, gridDim.z);",
+                "    ek_lo += (int)blockIdx.z * ek_per;",
+                "    ek_hi = ek::Min::op<int>(ek_hi, ek_lo + ek_per);",
+                "    if (blockIdx.z) {",
+                "      #pragma unroll",
+                f"      for (int r = 0; r < {n}; ++r) {nm}[r] = 0.0f;",
+                "    }",
+                "  }",
+                f"{run}ek_lo, ek_hi, ek_smem, ek_tid);",
+                f"  if (ek_ws && !ek::split_reduce<{n}, {self.nt}>({nm}, ek_ws, ek_smem, ek_tid)) "
+                "return;"]
+            serial = [
+                f"  ek::SliceSum<{n}> ek_sum({nm}, ek::split_slice({lo}, {hi}, {bk}, ek_ns) / {bk});",
+                f"{run}{lo}, {hi}, ek_smem, ek_tid, ek_sum);",
+                "  ek_sum.finish();"]
+            for ln in parallel:
+                self.emit(ln)
+            self.split_text = tuple("\n".join(ind + ln for ln in x) for x in (parallel, serial))
         self.emit("}")
         self.define(op.results[0], nm)
         self.big_acc = max(getattr(self, "big_acc", 0), lay.nregs)
@@ -3993,8 +4007,9 @@ class Emitter:
             params.append("uint32_t* ek_assert_buf")
             args.append(KernelArg("ek_assert_buf", "ptr", core.uint32, "uint32_t*"))
         if self.split:
-            params.append("float* ek_ws")
-            args.append(KernelArg("ek_ws", "ptr", core.float32, "float*"))
+            params += ["float* ek_ws", "int32_t ek_ns"]
+            args += [KernelArg("ek_ws", "ptr", core.float32, "float*"),
+                     KernelArg("ek_ns", "scalar", core.int32, "int32_t")]
         # Two-level flush of privatised bins: each workgroup stores its bins to a partial
         # buffer row (plain stores), and a second kernel sums a block of RB rows by 64 words
         # and adds each sum with one global atomic. Measured on the 1024-bin histogram: one
@@ -4124,6 +4139,14 @@ class Emitter:
                            "__HIP_MEMORY_SCOPE_AGENT);")
                 out.append("  }")
         out.append("}")
+        if self.split:
+            parallel, serial = self.split_text
+            text = "\n".join(out[2:])
+            assert text.count(parallel) == 1 and text.count(f" {kname}(") == 1
+            out += ["", "// The same for launches without a workspace: one workgroup per tile walks "
+                    "the ek_ns slices.",
+                    text.replace(parallel, serial).replace(f" {kname}(",
+                                                           f" {self.split['serial']}(")]
         flush = None
         if two:
             rb = int(self.opt.get("priv_flush_rows", 256))

@@ -845,6 +845,52 @@ struct GemmTile<float, BM, BN, BK, WM, WN, NT, TR> {
   }
 };
 
+// How a loop goes through its n steps: one after the other, or, where one workgroup takes the
+// slices of a split k loop in turn (see split_reduce), in slices of `per` steps: at each slice's
+// end the accumulator is added to the sum of those before and starts again from zero, so that
+// the result has the bits of slices computed apart. A loop that can runs up to `end` and
+// asks for `more` (fp16 64 x 4096 x 4096 at 64x64x128, captured: 22.7 us as one slice, 24.7
+// in 4, 25.7 with a test in each step; 512 x 512 x 8192 at 128x128x64: 83.4 and 83.2 in 15;
+// at 256x256x64, where accumulators and sums do not fit the registers, 145 and 203, and 446 with the
+// test). Otherwise it calls `begin` before each step.
+struct OneSlice {
+  EK_INLINE int end(int, int n) { return n; }
+  EK_INLINE bool more(int, int) { return false; }
+  EK_INLINE void begin(int) {}
+};
+template <int R> struct SliceSum {
+  float* acc;
+  float sum[R];
+  int per, next;
+  EK_INLINE SliceSum(float* acc_, int per_) : acc(acc_), per(per_), next(per_) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) sum[r] = 0.0f;
+  }
+  EK_INLINE void fold() {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      sum[r] += acc[r];
+      acc[r] = 0.0f;
+    }
+  }
+  EK_INLINE int end(int it, int n) { return Min::op<int>(next = it + per, n); }
+  EK_INLINE bool more(int it, int n) {
+    if (it == next) fold();
+    return it < n;
+  }
+  EK_INLINE void begin(int it) {
+    if (it == next) {
+      fold();
+      next += per;
+    }
+  }
+  EK_INLINE void finish() {
+    fold();
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = sum[r];
+  }
+};
+
 // ---------------------------------------------------------------------------
 // The loop for operands of any alignment and size, through registers: each thread loads its
 // 16-byte chunks of the tile PD steps ahead (element-aligned vector loads) and writes the tile
@@ -948,14 +994,15 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
   }
 
   // One element of an operand [rows, cols], zero outside it.
-  static EK_INLINE E at(const T* P, int64_t ld, int rows, int cols, int i, int j) {
+  static EK_INLINE E elem(const T* P, int64_t ld, int rows, int cols, int i, int j) {
     if (i < 0 || i >= rows || j < 0 || j >= cols) return 0;
     return reinterpret_cast<const E*>(P)[i * ld + j];
   }
 
   // Runs the whole k loop: k = lo, lo + BK, ... < hi.
+  template <typename At = OneSlice>
   EK_INLINE void run(float* acc, const T* A, int lda, const T* B, int ldb, int M, int N, int K,
-                     int m0, int n0, int lo, int hi, char* smem, int tid) {
+                     int m0, int n0, int lo, int hi, char* smem, int tid, At&& at = At{}) {
     hi = Min::op<int>(hi, K);   // past K both operands are zero
     if (hi <= lo) return;
     const int niter = (int)(((int64_t)hi - lo + BK - 1) / BK);
@@ -968,11 +1015,12 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
         const int k = lo + it * BK;
         for (int c = tid; c < BM * BK; c += NT)
           sm[G::a_chunk(c / BK, (c % BK) / EC) * EC + c % EC] =
-              at(A, lda, M, K, m0 + c / BK, k + c % BK);
+              elem(A, lda, M, K, m0 + c / BK, k + c % BK);
         for (int c = tid; c < BK * BN; c += NT)
           sm[A_ELEMS + G::b_chunk(c / BN, (c % BN) / EC) * EC + c % EC] =
-              at(B, ldb, K, N, k + c / BN, n0 + c % BN);
+              elem(B, ldb, K, N, k + c / BN, n0 + c % BN);
         __syncthreads();
+        at.begin(it);
         G::template compute<0, TK>(acc, sm, lane, wm, wn);
         __syncthreads();
       }
@@ -991,21 +1039,25 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
       const int t = Min::op<int>(p, niter - 1);
       load(p, a + t * sa, b + t * sb, t == niter - 1, tid);
     }
-    for (int it = 0; it < niter; it += PD) {
+    for (int it = 0, stop = PD == 1 ? at.end(0, niter) : niter;; stop = at.end(it, niter)) {
+      for (; it < stop; it += PD) {
 #pragma unroll
-      for (int p = 0; p < PD; ++p) {
-        const int t = it + p;
-        if (t >= niter) break;
-        const bool end = t == niter - 1;
-        if (edge || (end && ragged)) shift(p, end);
-        E* st = sm + (PD % 2 ? (t & 1) : (p & 1)) * STAGE;
-        put(p, st, tid);
-        // past the end: the last tile again, which nothing reads
-        const int nx = Min::op<int>(t + PD, niter - 1);
-        load(p, a + nx * sa, b + nx * sb, nx == niter - 1, tid);
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        G::template compute<0, TK>(acc, st, lane, wm, wn);
+        for (int p = 0; p < PD; ++p) {
+          const int t = it + p;
+          if (t >= niter) break;
+          const bool end = t == niter - 1;
+          if (edge || (end && ragged)) shift(p, end);
+          E* st = sm + (PD % 2 ? (t & 1) : (p & 1)) * STAGE;
+          put(p, st, tid);
+          // past the end: the last tile again, which nothing reads
+          const int nx = Min::op<int>(t + PD, niter - 1);
+          load(p, a + nx * sa, b + nx * sb, nx == niter - 1, tid);
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          if constexpr (PD > 1) at.begin(t);
+          G::template compute<0, TK>(acc, st, lane, wm, wn);
+        }
       }
+      if (PD > 1 || !at.more(it, niter)) break;
     }
     __syncthreads();
   }
@@ -1110,8 +1162,9 @@ struct GemmDma : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
   }
 
   // Runs the whole k loop: k = lo, lo + BK, ... < hi.
+  template <typename At = OneSlice>
   EK_INLINE void run(float* acc, const T* A, int lda, const T* B, int ldb, int M, int N, int K,
-                     int m0, int n0, int lo, int hi, char* smem, int tid) {
+                     int m0, int n0, int lo, int hi, char* smem, int tid, At&& at = At{}) {
     hi = Min::op<int>(hi, K);   // past K both operands are zero
     if (hi <= lo) return;
     const int niter = (hi - lo + BK - 1) / BK;
@@ -1139,31 +1192,34 @@ struct GemmDma : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
     __builtin_amdgcn_s_waitcnt(0x0F70);
 #pragma unroll
     for (int s = 0; s < S - 1; ++s) copy(ra, rb, ldb, K, lo + s * BK, l0 + s * STAGE * 2, wave);
-    for (int it = 0; it < nloop; ++it) {
-      // this wave's copies of stage `it` have landed (S - 2 younger stages may still fly),
-      // its reads of the previous stage are complete; then everyone's are.
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * D) : "memory");
-      // The first SPLIT k slices' fragment reads go out before any copy, so their latency
-      // hides behind the copy issue instead of stalling the first MFMA; the copies of the
-      // stage S - 1 ahead are then spread over the remaining slices, a share before each
-      // slice's reads, so each share's issue overlaps the MFMAs already queued (as one block
-      // the copies kept the wave from issuing for 500-800 cycles per k step).
-      const uint16_t* cur = s16 + (it % S) * STAGE;
-      G::template compute<0, SPLIT>(acc, cur, lane, wm, wn);
-      if constexpr (SPLIT < TK) {
-        constexpr int SL = TK - SPLIT, PER = (D + SL - 1) / SL;
-        const int kn = lo + (it + S - 1) * BK;
-        const uint32_t stn = l0 + ((it + S - 1) % S) * STAGE * 2;
+    for (int it = 0, stop = at.end(0, nloop);; stop = at.end(it, nloop)) {
+      for (; it < stop; ++it) {
+        // this wave's copies of stage `it` have landed (S - 2 younger stages may still fly),
+        // its reads of the previous stage are complete; then everyone's are.
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * D) : "memory");
+        // The first SPLIT k slices' fragment reads go out before any copy, so their latency
+        // hides behind the copy issue instead of stalling the first MFMA; the copies of the
+        // stage S - 1 ahead are then spread over the remaining slices, a share before each
+        // slice's reads, so each share's issue overlaps the MFMAs already queued (as one block
+        // the copies kept the wave from issuing for 500-800 cycles per k step).
+        const uint16_t* cur = s16 + (it % S) * STAGE;
+        G::template compute<0, SPLIT>(acc, cur, lane, wm, wn);
+        if constexpr (SPLIT < TK) {
+          constexpr int SL = TK - SPLIT, PER = (D + SL - 1) / SL;
+          const int kn = lo + (it + S - 1) * BK;
+          const uint32_t stn = l0 + ((it + S - 1) % S) * STAGE * 2;
 #pragma unroll
-        for (int q = 0; q < SL; ++q) {
+          for (int q = 0; q < SL; ++q) {
 #pragma unroll
-          for (int j = q * PER; j < (q + 1) * PER && j < D; ++j)
-            copy_one(j, ra, rb, ldb, K, kn, stn, wave);
-          G::compute_kk(SPLIT + q, acc, cur, lane, wm, wn);
+            for (int j = q * PER; j < (q + 1) * PER && j < D; ++j)
+              copy_one(j, ra, rb, ldb, K, kn, stn, wave);
+            G::compute_kk(SPLIT + q, acc, cur, lane, wm, wn);
+          }
+        } else {
+          copy(ra, rb, ldb, K, lo + (it + S - 1) * BK, l0 + ((it + S - 1) % S) * STAGE * 2, wave);
         }
-      } else {
-        copy(ra, rb, ldb, K, lo + (it + S - 1) * BK, l0 + ((it + S - 1) % S) * STAGE * 2, wave);
       }
+      if (!at.more(it, nloop)) break;
     }
     // drain the copies issued past the end before anyone reuses the LDS
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -1187,6 +1243,8 @@ struct GemmDma : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
 // as they are, NT lanes side by side) to its row of the workspace and counts itself in; the
 // last one of a tile adds all rows in slice order (so the sum does not depend on who is last),
 // clears the tile's counter for the next launch and returns true: it runs the epilogue.
+// Launches that find no workspace run one workgroup per tile, which walks the same slices in the
+// same order (SliceSum): whether a launch had a workspace shows in its time, not in its bits.
 //
 // The partial rows go through relaxed agent-scope atomics, which write to and read from memory
 // past the XCDs' private L2s; a vmcnt wait before the count makes sure that they are there. That

@@ -145,8 +145,10 @@ class CompiledKernel:
 
     def pack(self, values) -> bytes:
         values = list(values)
-        if self.gen.flush or self.gen.split:
-            values.append(0)      # the partial-bin buffer or workspace, set per stream at launch
+        if self.gen.flush:
+            values.append(0)      # the partial-bin buffer, set per stream at launch
+        if self.gen.split:
+            values += [0, 1]      # the workspace and the number of slices, set at launch
         b = codegen_hip.pack_args(self.args, values, pad8=not (self.gen.coarsen or self.gen.pack))
         self.packed_size = len(b)
         return b
@@ -159,6 +161,16 @@ class CompiledKernel:
                      ctypes.byref(f))
             self._flush_fn = f
         return self._flush_fn
+
+    def _serial_function(self):
+        """The function that walks the slices of a split k loop in one workgroup per tile."""
+        if getattr(self, "_serial_fn", None) is None:
+            self.function()
+            f = ctypes.c_void_p()
+            hip.call("ek_module_function", self._module, self.gen.split["serial"].encode(),
+                     ctypes.byref(f))
+            self._serial_fn = f
+        return self._serial_fn
 
     def _partials(self, stream: int, nwg: int) -> int:
         """The partial-bin buffer for launches on `stream` (kept for the kernel's life;
@@ -186,16 +198,22 @@ class CompiledKernel:
             kernarg += b"\0" * ((-len(kernarg)) % 8)
         out = []
         fl = self.gen.flush
+        fn = self.function()
         if self.gen.split and gz == 1:
             import struct
             offs = codegen_hip.arg_offsets(self.args)
             hi = struct.unpack_from("<i", kernarg, offs[self.gen.split["hi"]])[0]
             n = split_factor(self.gen.split, gx * gy, hi)
-            ws = workspace(stream) if n > 1 else 0
-            if ws:
+            if n > 1:
+                ws = workspace(stream)
                 kb = bytearray(kernarg)
-                struct.pack_into("<Q", kb, offs[-1], ws)
-                kernarg, gz = bytes(kb), n
+                struct.pack_into("<Q", kb, offs[-2], ws)
+                struct.pack_into("<i", kb, offs[-1], n)
+                kernarg = bytes(kb)
+                if ws:
+                    gz = n
+                else:
+                    fn = self._serial_function()
         if fl:
             import struct
             offs = codegen_hip.arg_offsets(self.args)
@@ -209,7 +227,7 @@ class CompiledKernel:
                 [codegen_hip.KernelArg("h", "ptr", None, "int32_t*") for _ in bases]
             fk = codegen_hip.pack_args(fargs, [part, gx, *bases])
         buf = ctypes.create_string_buffer(kernarg, len(kernarg))
-        out.append((self.function(), (gx, gy, gz), self.gen.block, buf, len(kernarg)))
+        out.append((fn, (gx, gy, gz), self.gen.block, buf, len(kernarg)))
         if fl:
             fbuf = ctypes.create_string_buffer(fk, len(fk))
             out.append((self._flush_function(), (fl["chunks"], (gx + fl["rb"] - 1) // fl["rb"], 1), 256,
@@ -269,9 +287,10 @@ class CompiledKernel:
                 hip.call("ek_launch", ctypes.c_void_p(stream or None), fn_, g_[0], g_[1],
                          g_[2], blk, 1, 1, 0, buf, n)
             if t0 is not None:
-                nm = self.name if fn_ is self._function else self.gen.flush["name"]
-                debug.after_launch(t0, stream, nm, g_, blk,
-                                   self.gen.lds_bytes if fn_ is self._function else 0)
+                second = fn_ is getattr(self, "_flush_fn", None)
+                nm = self.gen.flush["name"] if second else self.name if \
+                    fn_ is self._function else self.gen.split["serial"]
+                debug.after_launch(t0, stream, nm, g_, blk, 0 if second else self.gen.lds_bytes)
 
 
 _CAP = None
@@ -311,7 +330,7 @@ _ws_tls = threading.local()
 
 def workspace(stream: int) -> int:
     """The device address of `stream`'s split workspace, or 0 when it has none (captured
-    streams, too many streams): the launch then does not split."""
+    streams, too many streams): one workgroup per tile then walks the slices in turn."""
     t = _ws_tls
     if not hasattr(t, "ptr"):
         t.ptr, t.err = ctypes.c_void_p(), ctypes.create_string_buffer(1024)

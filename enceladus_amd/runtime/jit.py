@@ -702,6 +702,7 @@ class JITFunction:
             return None                 # `enceladus.capture` records the general path
         if stream is None:
             stream = _launch_stream()
+        fn = ent.fn
         if ent.split is not None:
             ws, n = 0, 1
             if gz == 1:
@@ -709,7 +710,9 @@ class JITFunction:
                 ws = C.workspace(stream) if n > 1 else 0
             if ws:
                 gz = n
-            rt.append(ws)
+            elif n > 1:
+                fn = ent.lc.ck._serial_function()
+            rt += (ws, n)
         flush = ent.flush
         if ent.pack:
             rt.append(gx)
@@ -728,14 +731,14 @@ class JITFunction:
             return None                 # a float beyond fp32's range: general packing
         t = _timing.current()
         if t is not None:
-            t.launch(stream, ent.fn, (gx, gy, gz), ent.block, kb, len(kb))
+            t.launch(stream, fn, (gx, gy, gz), ent.block, kb, len(kb))
             if flush is not None:
                 t.launch(stream, flush[0], (flush[3], -(-gx // flush[4]), 1), 256, second,
                          len(second))
             return ent.lc.ck
         err = _errbuf()
         launch = _ek_launch()
-        if launch(stream or None, ent.fn, gx, gy, gz, ent.block, 1, 1, 0, kb, len(kb), err,
+        if launch(stream or None, fn, gx, gy, gz, ent.block, 1, 1, 0, kb, len(kb), err,
                   1024) or flush is not None and \
                 launch(stream or None, flush[0], flush[3], -(-gx // flush[4]), 1, 256, 1, 1, 0,
                        second, len(second), err, 1024):

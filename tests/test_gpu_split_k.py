@@ -1,6 +1,6 @@
 """Block GEMM loops split along k over several workgroups per tile: exact against integer
 products (every partial sum is exact), the same bits on every launch, whole against sliced, on
-several streams and threads, and under graph capture (where they do not split)."""
+several streams and threads, and under graph capture (where one workgroup walks the slices)."""
 
 import threading
 
@@ -113,3 +113,82 @@ def test_captured_launches_do_not_split(monkeypatch):
         torch.cuda.synchronize()
         assert torch.equal(c, want)
         matmul_desc(a, b, bm=64, bn=64, bk=64)         # eager work between replays
+
+
+def _normal(rows, cols, seed, dtype):
+    import torch
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(rows, cols, generator=g).to(getattr(torch, dtype)).cuda()
+
+
+@pytest.mark.parametrize("dtype", ["float16", "float32"])
+@pytest.mark.parametrize("slices", [2, 3, 7])
+@pytest.mark.parametrize("mnk", [(64, 64, 512), (33, 70, 1000), (130, 264, 1024), (5, 3, 999)])
+def test_launches_without_a_workspace_have_the_same_bits(mnk, slices, dtype, monkeypatch):
+    """One workgroup per tile walks the slices in turn: same sums in the same order."""
+    import torch
+    m, n, k = mnk
+    a, b = _normal(m, k, 1, dtype), _normal(k, n, 2, dtype)
+    tiles = [(matmul_desc, 64, 64, 64, 4), (matmul, 64, 64, 32, 4), (matmul_desc, 128, 128, 32, 4)]
+    if dtype == "float16":
+        tiles.append((matmul_desc, 256, 256, 64, 8))
+    for f, bm, bn, bk, nw in tiles:
+        outs = []
+        for ws in (True, False):
+            with monkeypatch.context() as mp:
+                mp.setattr(C, "split_factor", lambda split, tiles, hi: slices)
+                if not ws:
+                    mp.setattr(C, "workspace", lambda stream: 0)
+                outs += [f(a, b, bm=bm, bn=bn, bk=bk, num_warps=nw) for _ in range(2)]
+        assert all(torch.equal(o, outs[0]) for o in outs), (f.__name__, bm, bn, bk)
+
+
+def test_broadcast_rows_without_a_workspace(monkeypatch):
+    """Rows of B that coincide: the ragged last step is the last slice's."""
+    import torch
+    _force(monkeypatch, 3)
+    a = _normal(64, 624, 1, "float16")
+    b = _normal(1, 128, 2, "float16").expand(624, 128)
+    want = matmul(a, b)
+    torch.testing.assert_close(want.double(), a.double() @ b.double(), rtol=2e-2, atol=2e-2)
+    monkeypatch.setattr(C, "workspace", lambda stream: 0)
+    assert torch.equal(matmul(a, b), want)
+
+
+@pytest.mark.parametrize("path", ["warm", "general"])
+def test_captured_and_late_streams_have_the_same_bits(path, tmp_path):
+    """A shape that the rule splits: eager, captured, and on more streams than have workspaces."""
+    import contextlib
+
+    import enceladus
+    import torch
+    a, b = _normal(64, 4096, 1, "float16"), _normal(4096, 512, 2, "float16") / 64
+    bias = _normal(1, 512, 3, "float16")[0]
+    out = torch.empty(64, 512, dtype=torch.float16, device="cuda")
+    traces = iter(range(100))
+
+    def call(o):
+        cm = enceladus.capture(str(tmp_path / f"{next(traces)}.json")) if path == "general" \
+            else contextlib.nullcontext()
+        with cm:
+            return matmul_bias_gelu(a, b, bias, o, bm=64, bn=64, bk=128)
+    want = call(torch.empty_like(out))
+    assert C.split_factor({"bk": 128, "words": 4096, "step_us": 0.655}, 8, 4096) > 1
+    streams = [torch.cuda.Stream() for _ in range(12)]
+    torch.cuda.synchronize()
+    for s in streams:
+        with torch.cuda.stream(s):
+            got = call(torch.empty_like(out))
+        s.synchronize()
+        assert torch.equal(got, want)
+    if path == "general":
+        return                                      # a dispatch trace waits for each launch
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        call(out)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        call(torch.empty_like(out))
