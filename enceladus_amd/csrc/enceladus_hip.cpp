@@ -211,6 +211,7 @@ int ek_stream_new(void** stream, char* err, size_t errlen) {
 int ek_workspace(void* stream, void** ptr, char* err, size_t errlen) {
   *ptr = nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (s == hipStreamPerThread) return 0;   // one handle for a stream of each thread
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || hipStreamIsCapturing(s, &cap) != hipSuccess ||
@@ -225,16 +226,27 @@ int ek_workspace(void* stream, void** ptr, char* err, size_t errlen) {
     return 0;
   }
   if (g_ws.size() >= EK_WORKSPACES) return 0;
-  void* p = nullptr;
-  if (hipMalloc(&p, EK_WORKSPACE_BYTES) != hipSuccess) {
+  // An allocation is a call that another thread's capture (in the global mode) forbids, and that
+  // would end that capture, unless this thread's calls are exempt from it. Nothing waits for the
+  // device: the counters start at zero in the stream's order, and every launch leaves them there.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
-  // the counters start at zero, and every launch leaves them there
-  if (hipMemset(p, 0, EK_WORKSPACE_BYTES) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+  void* p = nullptr;
+  bool ok = hipMalloc(&p, EK_WORKSPACE_BYTES) == hipSuccess;
+  if (ok && hipMemsetAsync(p, 0, EK_WORKSPACE_BYTES, s) != hipSuccess) {
     (void)hipFree(p);
-    return fail(err, errlen, "ek_workspace: clearing the workspace failed");
+    ok = false;
   }
+  if (!ok) (void)hipGetLastError();
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+    if (ok) (void)hipFree(p);
+    (void)hipGetLastError();
+    return fail(err, errlen, "ek_workspace: the thread's capture mode could not be restored");
+  }
+  if (!ok) return 0;
   g_ws[{dev, s}] = p;
   *ptr = p;
   return 0;

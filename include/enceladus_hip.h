@@ -138,11 +138,13 @@ int ek_launch_flush_noalloc(void* stream, void* function, uint32_t gx, uint32_t 
 /* No counterpart in the reference. The workspace of launches that split a k loop over several
  * workgroups per tile (a float row per workgroup, after 16384 tile counters that are zero between
  * launches): EK_WORKSPACE_BYTES of device memory kept for `stream` on the current device, made
- * by the first call. Launches in one stream's order share it. Sets *ptr to NULL, and the caller
- * launches without splitting, when the stream is being captured into a graph (replays on other
- * streams would race on the workspace), when EK_WORKSPACES streams have one already, or when
- * there is no memory. ek_stream_free gives a stream's workspace back; ek_workspace_release
- * all of them, once their devices are idle (no split launch may be in preparation). */
+ * by the first call (which waits for nothing, and is allowed beside another thread's capture).
+ * Launches in one stream's order share it. Sets *ptr to NULL, and the caller launches the
+ * kernel's serial function, when the stream is being captured into a graph (replays on other
+ * streams would race on the workspace), when it is hipStreamPerThread (one handle for many
+ * streams), when EK_WORKSPACES streams have one already, or when there is no memory.
+ * ek_stream_free gives a stream's workspace back; ek_workspace_release all of them, once their
+ * devices are idle (no split launch may be in preparation). */
 #define EK_WORKSPACE_BYTES (16u << 20)
 #define EK_WORKSPACES 8
 int ek_workspace(void* stream, void** ptr, char* err, size_t errlen);

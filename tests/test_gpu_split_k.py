@@ -192,3 +192,47 @@ def test_captured_and_late_streams_have_the_same_bits(path, tmp_path):
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         call(torch.empty_like(out))
+
+
+def test_first_split_launch_beside_another_threads_capture(monkeypatch):
+    """A stream's workspace is made by its first split launch, also while another thread captures
+    (in the global mode, which forbids allocations): neither disturbs the other."""
+    import torch
+    from enceladus_amd.runtime import hip
+    _force(monkeypatch, 4)
+    a, b = whole(64, 4096, 1, 0), whole(4096, 128, 2, 0)
+    c, d = (torch.zeros(64, 128, dtype=torch.float16, device="cuda") for _ in range(2))
+    want = a.double() @ b.double()
+    matmul_desc(a, b, c, bm=64, bn=64, bk=64)            # compiled and loaded
+    side, own = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    hip.call("ek_workspace_release")                      # no stream has one
+    seen, errors = [], []
+    real = C.workspace
+    monkeypatch.setattr(C, "workspace", lambda st: seen.append(real(st)) or seen[-1])
+
+    def launch():
+        try:
+            with torch.cuda.stream(own):
+                matmul_desc(a, b, d, bm=64, bn=64, bk=64)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side, capture_error_mode="global"):
+        matmul_desc(a, b, c, bm=64, bn=64, bk=64)
+        t = threading.Thread(target=launch)
+        t.start()
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors and seen[0] == 0 and seen[1] != 0
+    assert torch.equal(d.double(), want)
+    for _ in range(3):
+        c.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c.double(), want)
+
+
+def test_the_per_thread_stream_has_no_workspace():
+    """hipStreamPerThread is one handle for a stream of each thread, which are not ordered."""
+    assert C.workspace(2) == 0
