@@ -236,3 +236,14 @@ def test_first_split_launch_beside_another_threads_capture(monkeypatch):
 def test_the_per_thread_stream_has_no_workspace():
     """hipStreamPerThread is one handle for a stream of each thread, which are not ordered."""
     assert C.workspace(2) == 0
+
+
+def test_large_accumulators_split_less():
+    """One workgroup reads all rows of its tile: 256x256 tiles (256 KB a row) take fewer slices
+    than 128x128 ones of the same loop, and none where the unsplit loop is as fast."""
+    big, mid = ({"bk": 64, "words": w, "step_us": st} for w, st in ((65536, 1.71), (16384, 0.655)))
+    assert C.split_factor(big, 4, 1024) == 1          # 22.8 us unsplit, 27.7 over 2, 34.2 over 5
+    assert 2 < C.split_factor(big, 4, 2048) < 6       # 38.7, 34.4 over 3, 54.3 over 10
+    assert 4 < C.split_factor(big, 4, 8192) < 10      # 143.9, 58.5 over 8, 74.8 over 15
+    assert 4 < C.split_factor(mid, 16, 8192) < 12     # 84.8, 26.8 over 8, 32.9 over 15
+    assert C.split_factor(big, 4, -64) == 1
