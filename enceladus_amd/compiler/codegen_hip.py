@@ -1776,7 +1776,8 @@ class Emitter:
         rank = op.result.type.rank
         info = {"base": self.name[base.id], "shape": vals[:rank], "strides": vals[rank:],
                 "base_v": base, "shape_v": op.operands[1:1 + rank],
-                "stride_v": op.operands[1 + rank:]}
+                "stride_v": op.operands[1 + rank:],
+                "any_row_stride": bool(op.attrs.get("any_row_stride"))}
         self.desc[op.result.id] = info
         self.def_level[op.result.id] = len(self.scopes) - 1
 
@@ -3322,8 +3323,13 @@ class Emitter:
 
     def _stage_buffer_ok(self, info, d, W: int) -> bool:
         """Whether a stage can load through raw buffer loads: 32-bit byte offsets, aligned
-        rows, and column chunks of W elements that lie wholly inside or outside the tile."""
-        if self.opt.get("no_buffer_loads") or d["base_v"].facts.get("span2g"):
+        rows, and column chunks of W elements that lie wholly inside or outside the tile. The
+        resources end after rows x row stride and reject rows past the last by address, which
+        holds for rows that do not overlap: descriptors made from pointer loops, whose row
+        stride may be anything (0, shorter than the row, negative), load with 64-bit addresses
+        and tests."""
+        if self.opt.get("no_buffer_loads") or d["base_v"].facts.get("span2g") or \
+                d["any_row_stride"]:
             return False
         div = lambda v: self.axis.get(v).div[0]  # noqa: E731
         if div(d["base_v"]) < 2 * W or div(d["stride_v"][0]) % W:

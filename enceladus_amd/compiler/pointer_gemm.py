@@ -497,7 +497,8 @@ class _Loop:
                 base.facts["span2g"] = True       # (a base of unknown origin may span as much)
             strides = [self.poly(p["stride"]), self.iconst(1)]
             d = self.emit("make_desc", [base, *shape, *strides],
-                          [ir.DescType(p["dtype"], tuple(p["shape"]))])
+                          [ir.DescType(p["dtype"], tuple(p["shape"]))],
+                          {"any_row_stride": True})
             ld = p["load"]
             new = ir.Op("desc_load", [d, *offs], [ld.result.type], loc=ld.loc)
             repl[id(ld)] = new

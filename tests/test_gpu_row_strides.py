@@ -47,14 +47,14 @@ SIZES = [(64, 64, 64), (100, 96, 208), (130, 264, 528), (37, 83, 101), (65, 90, 
 TILES = [(64, 64, 32, 4), (128, 128, 64, 4), (256, 128, 64, 8)]
 
 
-def check(mnk, tile, sa, sb, dtype="float16"):
+def check(mnk, tile, sa, sb, dtype="float16", forms=(True, False)):
     import torch
     m, n, k = mnk
     bm, bn, bk, nw = tile
     a, av = rows(m, k, sa, 1, dtype)
     b, bv = rows(k, n, sb, 2, dtype)
     want = av @ bv
-    for pointers in (True, False):
+    for pointers in forms:
         c = torch.full((m, n), 7.0, dtype=torch.float32, device="cuda")
         grid = (enceladus.cdiv(n, bn), enceladus.cdiv(m, bm))
         if pointers:
@@ -99,3 +99,15 @@ def test_descending_rows(mnk, dtype):
         for sb in (-n, -(n + 24), -16, -3):
             check(mnk, tile, k, sb, dtype)
         check(mnk, tile, -k, -(n + 8), dtype)
+
+
+@pytest.mark.parametrize("tile", [(32, 32, 32, 4), (64, 64, 32, 8), (32, 64, 64, 8),
+                                  (128, 32, 32, 8)])
+@pytest.mark.parametrize("mnk", SIZES[:3] + SIZES[4:])
+def test_pointer_loops_of_tiles_that_go_through_stages(mnk, tile):
+    """Tiles the block GEMM loops do not take: their operands are staged one by one."""
+    m, n, k = mnk
+    for sa in (0, 16, k - 16, k, -k, -(k + 24), -3):
+        check(mnk, tile, sa, n, forms=(True,))
+    for sb in (0, 16, n - 16, n + 24, -n, -(n + 24), -3):
+        check(mnk, tile, k, sb, forms=(True,))
