@@ -3328,9 +3328,11 @@ class Emitter:
         holds for rows that do not overlap: descriptors made from pointer loops, whose row
         stride may be anything (0, shorter than the row, negative), load with 64-bit addresses
         and tests."""
-        if self.opt.get("no_buffer_loads") or d["base_v"].facts.get("span2g") or \
-                d["any_row_stride"]:
-            return False
+        return not (self.opt.get("no_buffer_loads") or d["base_v"].facts.get("span2g") or
+                    d["any_row_stride"]) and self._stage_rows_aligned(info, d, W)
+
+    def _stage_rows_aligned(self, info, d, W: int) -> bool:
+        """Whether every row of a stage's tile is whole chunks of W elements."""
         div = lambda v: self.axis.get(v).div[0]  # noqa: E731
         if div(d["base_v"]) < 2 * W or div(d["stride_v"][0]) % W:
             return False
@@ -3711,6 +3713,8 @@ class Emitter:
         it = ctype(iv.type.dtype)
         ivn = self.fresh("iv")
         stg = self.stage_loops.get(id(op), []) if hasattr(self, "stage_loops") else []
+        if op.attrs.get("lifted") and not self._lift_pays(op, stg):
+            self.report["undo_lift"] = op.loc
         dma = bool(stg) and all(self._stage_dma_ok(info) for info in stg)
         if dma:
             li = self.counter
@@ -3838,6 +3842,20 @@ class Emitter:
             self.emit('asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\\n\\ts_barrier" ::: "memory");')
         for r, nm in zip(op.results, names):
             self.define(r, nm)
+
+    def _lift_pays(self, op, stg) -> bool:
+        """Whether a pointer loop that was rewritten to descriptor loads and that the block GEMM
+        template does not take (fp32 tiles past the LDS, tiles of several waves to a 32x32 block)
+        is faster so. fp32 loops, which are not staged, are not: 2048^3 at 64x64x256 411 us through
+        pointers, 478 through descriptors. Staged 16-bit ones are where rows start on
+        16 bytes: 2048^3 at 64x64x64 on 8 waves 100 and 64 us, at 32x64x32 on 4 167 and 106; on
+        other rows only wide tiles of long steps are: 1000 x 3000 x 2000 at 32x64x64 128 and 97
+        us, but at 64x64x32 on 8 waves 129 and 172, at 64x32x64 75 and 96."""
+        if len(stg) != 2:
+            return False
+        a, b = (info["op"].result.type.shape for info in stg)
+        return all(self._stage_rows_aligned(i, self.desc[i["op"].operands[0].id], 8)
+                   for i in stg) or (a[1] >= 64 and b[1] > a[0])
 
     def _general_for(self, op):
         """Python `range` with a runtime or negative step: the trip count is computed once

@@ -516,6 +516,7 @@ class _Loop:
         body.ops[-1].operands = [self.dot.result]
         body.args = [self.iv, self.acc]
         op.operands = [*op.operands[:3], op.operands[2 + keep]]
+        op.attrs["lifted"] = True
         res = op.results[keep - 1]
         res.index = 0
         op.results = [res]

@@ -387,9 +387,12 @@ def build_module(jfn, arg_types, arg_facts, constexprs, num_warps, options) -> i
         verify.maybe_verify(fn, "the attention scale rewrite")
     ir.dce(fn)
     verify.maybe_verify(fn, "dead-code elimination")
-    if lifted and codegen_hip.generate(fn, options).lds_bytes > codegen_hip.MAX_LDS:
-        # Two LDS stages of such tiles do not fit (fp16 256x128x128): the loop as written
-        # needs LDS for one tile at a time, in passes where that does not fit either.
-        return build_module(jfn, arg_types, arg_facts, constexprs, num_warps,
-                            {**(options or {}), "no_pointer_gemm": True})
+    if lifted:
+        # Not where two LDS stages of the tiles do not fit (fp16 256x128x128: the loop as written
+        # needs LDS for one tile at a time, in passes where that does not fit either), nor
+        # where the emitter knows the loop as written to be the faster one.
+        gen = codegen_hip.generate(fn, options)
+        if gen.lds_bytes > codegen_hip.MAX_LDS or "undo_lift" in gen.report:
+            return build_module(jfn, arg_types, arg_facts, constexprs, num_warps,
+                                {**(options or {}), "no_pointer_gemm": True})
     return fn

@@ -106,7 +106,7 @@ def test_tiles_whose_stages_do_not_fit_stay(tile, mnk):
 
 def test_tiles_whose_stages_fit_are_lifted():
     from examples.matmul import matmul_kernel
-    for bm, bn, bk, nw in ((64, 64, 256, 8), (256, 256, 64, 8), (128, 128, 128, 4)):
+    for bm, bn, bk, nw in ((64, 64, 256, 4), (256, 256, 64, 8), (128, 128, 128, 4)):
         names = [op.name for op in ir.walk(matmul_kernel.ir(
             H, H, H, 1000, 3000, 2000, 2000, 1, 3000, 1, 3000, 1, BM=bm, BN=bn, BK=bk,
             num_warps=nw).body)]
@@ -147,3 +147,20 @@ def test_operands_stored_by_tile_are_described_tile_by_tile(kind):
     a, b = loads
     assert b.operands[2].op.name == "const" and b.operands[2].op.attrs["value"] == 0
     assert a.operands[1].op.name != "const"
+
+
+@pytest.mark.parametrize("tile,dtype,mnk,lifted", [
+    ((64, 64, 64, 8), "float16", (1024, 1024, 1024), True),     # staged, aligned rows
+    ((64, 64, 64, 8), "float16", (1000, 3000, 2000), False),
+    ((32, 64, 64, 4), "float16", (1000, 3000, 2000), True),     # wide tiles of long steps
+    ((32, 64, 32, 4), "float16", (1000, 3000, 2000), False),
+    ((64, 64, 256, 4), "float32", (1024, 1024, 1024), False),   # fp32 loops are not staged
+    ((64, 64, 32, 4), "float32", (1000, 3000, 2000), True),     # the block GEMM loops take any
+    ((64, 64, 32, 4), "float16", (999, 3001, 2001), True)])
+def test_loops_are_lifted_where_that_is_faster(tile, dtype, mnk, lifted):
+    from examples.matmul import matmul_kernel
+    (bm, bn, bk, nw), (m, n, k) = tile, mnk
+    x = np.zeros(16, dtype)
+    names = [op.name for op in ir.walk(matmul_kernel.ir(
+        x, x, x, m, n, k, k, 1, n, 1, n, 1, BM=bm, BN=bn, BK=bk, num_warps=nw).body)]
+    assert ("desc_load" in names) == lifted
