@@ -174,14 +174,17 @@ _FMT = {"int32_t": ("i", 4), "int64_t": ("q", 8), "uint32_t": ("I", 4), "uint64_
 class _FastEntry:
     """A specialization's pre-packed launch: kernarg struct, function, block size; how its k
     loop may split; for a coarsened program walk, the workgroups its grid is capped at; the
-    programs each workgroup runs (0: one); for a two-level flush, the second kernel's (function, kernarg struct, argument indices of the
-    flushed arrays, column chunks, rows per workgroup)."""
+    programs each workgroup runs (0: one); for a two-level flush, the second kernel's (function,
+    kernarg struct, argument indices of the flushed arrays, column chunks, rows per workgroup).
+    `plain`: none of these, one program per workgroup of the grid as it is (at most one of
+    them applies: only coarsened kernels flush, and those neither split nor pack)."""
 
-    __slots__ = ("lc", "st", "fn", "block", "split", "cap", "flush", "pack")
+    __slots__ = ("lc", "st", "fn", "block", "split", "cap", "flush", "pack", "plain")
 
     def __init__(self, lc, st, fn, block, split, cap, flush, pack):
         self.lc, self.st, self.fn, self.block = lc, st, fn, block
         self.split, self.cap, self.flush, self.pack = split, cap, flush, pack
+        self.plain = not (split or cap or flush or pack)
 
 
 def _fast_entry(lc) -> "_FastEntry | None":
@@ -702,8 +705,10 @@ class JITFunction:
             return None                 # `enceladus.capture` records the general path
         if stream is None:
             stream = _launch_stream()
-        fn = ent.fn
-        if ent.split is not None:
+        fn, flush = ent.fn, None
+        if ent.plain:
+            pass
+        elif ent.split is not None:
             ws, n = 0, 1
             if gz == 1:
                 n = C.split_factor(ent.split, gx * gy, rt[ent.split["hi"]])
@@ -713,11 +718,11 @@ class JITFunction:
             elif n > 1:
                 fn = ent.lc.ck._serial_function()
             rt += (ws, n)
-        flush = ent.flush
-        if ent.pack:
+        elif ent.pack:
             rt.append(gx)
             gx = -(-gx // ent.pack)
-        elif ent.cap:
+        else:                           # a coarsened walk, perhaps with a second flush kernel
+            flush = ent.flush
             logical = (gx, gy, gz)
             gx, gy, gz = min(gx * gy * gz, ent.cap), 1, 1
             if flush is not None:

@@ -342,10 +342,12 @@ def element_strides(obj: Any) -> tuple[int, ...]:
 
 def new_empty(like: Any, shape=None, dtype=None):
     """An uninitialised array of `like`'s kind (NumPy, torch, Tensor) and device."""
-    torch = sys.modules.get("torch")
-    if shape is None and dtype is None and torch is not None and type(like) is torch.Tensor:
-        # half the time of torch.empty with a shape
-        return torch.empty_like(like, memory_format=torch.contiguous_format)
+    if shape is None:
+        torch = sys.modules.get("torch")
+        if torch is not None and type(like) is torch.Tensor:
+            # half the time of torch.empty with a shape
+            return torch.empty_like(like, dtype=None if dtype is None else _torch_dtype(dtype),
+                                    memory_format=torch.contiguous_format)
     shape = tuple(like.shape) if shape is None else tuple(shape)
     if _is_torch(like):
         import torch
