@@ -165,7 +165,7 @@ class GeneratedKernel:
     pack: int = 0          # programs (along grid x) per workgroup (0: one)
     # a block GEMM that may be split along k: {"hi" (index of the argument that bounds k), "bk",
     # "words" (floats of one workgroup's accumulator), "step_us" (a k step's time, roughly),
-    # "serial" (the function for launches without a workspace)}; its last arguments are the
+    # "wait_us" (the same where its loads' latency is in sight), "serial" (the function for launches without a workspace)}; its last arguments are the
     # workspace (0: not split) and the number of slices, and a split launch runs one workgroup per
     # tile and slice (grid z), or the serial function with one workgroup per tile
     split: dict | None = None
@@ -3646,10 +3646,14 @@ class Emitter:
             # MB (64x64x128 fp16: 0.65 us measured), or its MFMAs at half their peak
             # (128x128x64 fp32: 5.2 us)
             rate = 0.4e6 if g["dt"] is core.float32 else 4.9e6
-            self.split = {"serial": f"ek_{self.fn.name}_serial", "hi": next(i for i, a in enumerate(self.fn.args)
-                                     if a is op.operands[1]), "bk": bk,
-                          "words": lay.nregs * self.nt,
-                          "step_us": round(max(2e-5 * stage, 2 * bm * bn * bk / rate), 3)}
+            step = max(2e-5 * stage, 2 * bm * bn * bk / rate)
+            self.split = {"serial": f"ek_{self.fn.name}_serial", "bk": bk,
+                          "hi": next(i for i, a in enumerate(self.fn.args)
+                                     if a is op.operands[1]),
+                          "words": lay.nregs * self.nt, "step_us": round(step, 3),
+                          # (what a step through registers takes: the latency of its loads)
+                          "wait_us": round(step if dma or g["dt"] is core.float32
+                                           else max(step, 2.7), 3)}
         run = (f"  ek_g.run({nm}, {A['base']}, {A['strides'][0]}, {B['base']}, "
                f"{B['strides'][0]}, {A['shape'][0]}, {B['shape'][1]}, {kend}, "
                f"{self.name[g['m0'].id]}, {self.name[g['n0'].id]}, ")
