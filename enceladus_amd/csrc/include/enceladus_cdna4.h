@@ -1063,14 +1063,14 @@ struct GemmReg : GemmTile<T, BM, BN, BK, WM, WN, NT, TR> {
   }
 };
 
-// Operands whose rows are known to start on 16 bytes (K or N are not whole chunks): only the
-// chunks moved at an edge are unaligned.
+// The same loop, named so in kernels whose operands' rows are known to start on 16 bytes (K or N,
+// or the tile's origin, are no whole chunks): only the chunks moved at an edge are unaligned there.
 template <typename T, int BM, int BN, int BK, int WM, int WN, int NT, bool BIG, bool TR = false>
 using Gemm = GemmReg<T, BM, BN, BK, WM, WN, NT, BIG, TR>;
 
 // ---------------------------------------------------------------------------
 // GEMM main loop fed by LDS DMA: C[BM x BN] += A[BM x K] * B[K x BN], 16-bit row-major
-// operands, fp32 accumulators in the 32x32x16 MFMA layout (same as Gemm).
+// operands, fp32 accumulators in the 32x32x16 MFMA layout (GemmTile).
 //
 //  - Tiles move global -> LDS with buffer_load ... lds (16 bytes per lane, no VGPRs): the 64
 //    lanes of one instruction fill 64 consecutive 16-byte LDS chunks, so each lane fetches

@@ -143,12 +143,14 @@ def test_launches_without_a_workspace_have_the_same_bits(mnk, slices, dtype, mon
         assert all(torch.equal(o, outs[0]) for o in outs), (f.__name__, bm, bn, bk)
 
 
-def test_broadcast_rows_without_a_workspace(monkeypatch):
-    """Rows of B that coincide: the ragged last step is the last slice's."""
+@pytest.mark.parametrize("k", [624, 272, 160])
+def test_broadcast_rows_without_a_workspace(k, monkeypatch):
+    """Rows of B that coincide: the ragged last step, which runs after the loop, ends the last
+    slice (10 steps of 64 in slices of 4) or is all of it (5 in slices of 2, 3 in slices of 1)."""
     import torch
     _force(monkeypatch, 3)
-    a = _normal(64, 624, 1, "float16")
-    b = _normal(1, 128, 2, "float16").expand(624, 128)
+    a = _normal(64, k, 1, "float16")
+    b = _normal(1, 128, 2, "float16").expand(k, 128)
     want = matmul(a, b)
     torch.testing.assert_close(want.double(), a.double() @ b.double(), rtol=2e-2, atol=2e-2)
     monkeypatch.setattr(C, "workspace", lambda stream: 0)
