@@ -14,8 +14,9 @@ Lowered as written, every step computes a pointer and a mask per element, loads 
 registers with a branch per vector, and moves both tiles to the MFMA layouts through LDS with
 two barriers each and no overlap. `lift_pointer_gemm` proves that such a loop reads two
 row-major blocks, zero outside a box, and replaces the loads with descriptor loads, which the
-emitter's block GEMM loops take: bf16 1000 x 3000 x 2000 at 64x64x32 went from 85.3 us
-to 36.5 us.
+emitter's block GEMM loops take: bf16 1000 x 3000 x 2000 at 64x64x32 takes 30.6 us so, and 86 as
+written. Row strides may be anything: 0, shorter than the row, negative. The caller undoes the
+rewrite where it does not fit or does not pay (`build_module`).
 
 The proof works on index tiles as polynomials: `sum_d coef_d * i_d + offset`, where i_d is the
 tile coordinate along dimension d and the coefficients and the offset are integer polynomials in

@@ -850,9 +850,9 @@ struct GemmTile<float, BM, BN, BK, WM, WN, NT, TR> {
 // end the accumulator is added to the sum of those before and starts again from zero, so that
 // the result has the bits of slices computed apart. A loop that can runs up to `end` and
 // asks for `more` (fp16 64 x 4096 x 4096 at 64x64x128, captured: 22.7 us as one slice, 24.7
-// in 4, 25.7 with a test in each step; 512 x 512 x 8192 at 128x128x64: 83.4 and 83.2 in 15;
-// at 256x256x64, where accumulators and sums do not fit the registers, 145 and 203, and 446 with the
-// test). Otherwise it calls `begin` before each step.
+// in 4, 25.7 with a test in each step; 512 x 512 x 8192 at 128x128x64: 83.4 and 82.9 in 7; at
+// 256x256x64, where accumulators and sums do not fit the registers, 145 and 174 in 7).
+// Otherwise it calls `begin` before each step.
 struct OneSlice {
   EK_INLINE int end(int, int n) { return n; }
   EK_INLINE bool more(int, int) { return false; }

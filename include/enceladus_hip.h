@@ -143,8 +143,9 @@ int ek_launch_flush_noalloc(void* stream, void* function, uint32_t gx, uint32_t 
  * kernel's serial function, when the stream is being captured into a graph (replays on other
  * streams would race on the workspace), when it is hipStreamPerThread (one handle for many
  * streams), when EK_WORKSPACES streams have one already, or when there is no memory.
- * ek_stream_free gives a stream's workspace back; ek_workspace_release all of them, once their
- * devices are idle (no split launch may be in preparation). */
+ * ek_stream_free gives a stream's workspace back (a stream that is destroyed by other means is
+ * synchronised first: its handle, and with it the workspace, may return); ek_workspace_release
+ * all of them, once their devices are idle (no split launch may be in preparation). */
 #define EK_WORKSPACE_BYTES (16u << 20)
 #define EK_WORKSPACES 8
 int ek_workspace(void* stream, void** ptr, char* err, size_t errlen);
