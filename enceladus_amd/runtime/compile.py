@@ -318,9 +318,10 @@ def split_factor(split: dict, tiles: int, hi: int) -> int:
     4). One workgroup reads all rows of its tile at the end, so that the whole is about
     loop / n + n * row, with a row of 64 KB (128x128) at 1.3 us and one of 256 KB at 4: n is at
     most where that is least (a 16-bit step through registers waits for its loads, 2.7 us: bf16
-    2 x 168 x 5039 at 128x128x64 216 us unsplit, 27.0 over 10, 30.6 over 6), and at least 3 (fp16 512 x 512 x K, 256x256x64: K = 1024 22.8 us
-    unsplit, 27.7 over 2; K = 2048 38.7, 34.4 over 3, 54.3 over 10; K = 8192 143.9, 58.5 over 8,
-    74.8 over 15; 128x128x64: K = 8192 84.8, 26.8 over 8, 32.9 over 15). The rows have to fit
+    2 x 168 x 5039 at 128x128x64 216 us unsplit, 27.0 over 10, 30.6 over 6), and at least 3
+    (fp16 512 x 512 x K, 256x256x64: K = 1024 22.8 us unsplit, 27.7 over 2; K = 2048 38.7, 34.4
+    over 3, 54.3 over 10; K = 8192 143.9, 58.5 over 8, 74.8 over 15; 128x128x64: K = 8192 84.8,
+    26.8 over 8, 32.9 over 15). The rows have to fit
     the workspace."""
     cus = coarsen_cap()
     if 2 * tiles > cus or tiles <= 0:
